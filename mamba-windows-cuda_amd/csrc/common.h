@@ -105,19 +105,22 @@ template <int K> __device__ __forceinline__ void buf_st_f32(rsrc_t r, uint32_t o
 // Dropping a wave's priority as it passes 1/2, 3/4 and 7/8 of its chunks lets the ones behind
 // catch up, so they finish close together.
 struct ProgressPrio {
-    int b1, b2, b3;  // chunks done at which the priority drops to 2, 1, 0
+    int next, b2, b3;  // chunks done at which the priority next drops; the later drops
     __device__ __forceinline__ explicit ProgressPrio(int nchunks)
-        : b1(nchunks / 2), b2(3 * nchunks / 4), b3(7 * nchunks / 8) {
+        : next(nchunks / 2), b2(3 * nchunks / 4), b3(7 * nchunks / 8) {
         __builtin_amdgcn_s_setprio(3);
     }
     __device__ __forceinline__ void update(int done) {
-        if (done == b1 || done == b2 || done == b3) {
-            if (done == b3)
-                __builtin_amdgcn_s_setprio(0);
-            else if (done == b2)
-                __builtin_amdgcn_s_setprio(1);
-            else
-                __builtin_amdgcn_s_setprio(2);
+        if (__builtin_expect(done != next, 1)) return;  // one compare per chunk
+        if (done >= b3) {
+            __builtin_amdgcn_s_setprio(0);
+            next = -1;
+        } else if (done >= b2) {
+            __builtin_amdgcn_s_setprio(1);
+            next = b3;
+        } else {
+            __builtin_amdgcn_s_setprio(2);
+            next = b2;
         }
     }
 };
