@@ -47,26 +47,29 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);
 }
-template <typename T> __device__ __forceinline__ float buf_ld(rsrc_t r, uint32_t off);
-template <> __device__ __forceinline__ float buf_ld<float>(rsrc_t r, uint32_t off) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+// A value as loaded, its conversion deferred to raw_f. 16-bit values stay in the 32-bit register that the load
+// fills: held as 16-bit values over a loop's back edge, the compiler may pack the loads of a prefetched tile in
+// pairs right after issuing them, which waits for the memory there.
+template <typename T> struct raw_of { typedef uint32_t type; };
+template <> struct raw_of<float> { typedef float type; };
+template <typename T> using raw_t = typename raw_of<T>::type;
+template <typename T> __device__ __forceinline__ raw_t<T> buf_raw(rsrc_t r, uint32_t off) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    else
+        return (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
 }
-template <> __device__ __forceinline__ float buf_ld<half_t>(rsrc_t r, uint32_t off) {
-    return static_cast<float>(__builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0)));
+template <typename T> __device__ __forceinline__ raw_t<T> raw_ld(const T* p) {
+    if constexpr (sizeof(T) == 4)
+        return *p;
+    else
+        return *reinterpret_cast<const uint16_t*>(p);
 }
-template <> __device__ __forceinline__ float buf_ld<bf16_t>(rsrc_t r, uint32_t off) {
-    return static_cast<float>(__builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0)));
-}
-// Raw storage-type load (conversion deferred, keeps fp16 values in 16 bits while in flight).
-template <typename T> __device__ __forceinline__ T buf_raw(rsrc_t r, uint32_t off);
-template <> __device__ __forceinline__ float buf_raw<float>(rsrc_t r, uint32_t off) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-template <> __device__ __forceinline__ half_t buf_raw<half_t>(rsrc_t r, uint32_t off) {
-    return __builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
-}
-template <> __device__ __forceinline__ bf16_t buf_raw<bf16_t>(rsrc_t r, uint32_t off) {
-    return __builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+template <typename T> __device__ __forceinline__ float raw_f(raw_t<T> v) {
+    if constexpr (sizeof(T) == 4)
+        return v;
+    else
+        return static_cast<float>(__builtin_bit_cast(T, (uint16_t)v));
 }
 template <typename T> __device__ __forceinline__ void buf_st(rsrc_t r, uint32_t off, float v);
 template <> __device__ __forceinline__ void buf_st<float>(rsrc_t r, uint32_t off, float v) {

@@ -105,22 +105,24 @@ __global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A
     const int64_t base = seq * L * ncols + (cvalid ? col : ncols - 1);
     const int p0 = lt * kTileSteps + r * RUN;
 
-    // position p -> time index t (the adjoint runs from the end)
+    // Position p -> step t (the adjoint runs from the end). Rows past the ends are read from the nearest row of the
+    // sequence and set to 0 afterwards: 16-bit loads under a branch were converted, and so waited for, one by one there
+    // ((4, 65536, 1024) fp16: 1140 us against 431, the adjoint 1491 against 573; fp32 adjoint 1178 against 1038).
+    raw_t<T> wa[RUN], wx[RUN], wh[REV ? RUN : 1];
+    auto row = [&](int t) { return base + (int64_t)max(0, min(t, L - 1)) * ncols; };
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) {
+        const int t = REV ? L - 1 - p0 - i : p0 + i;
+        wa[i] = raw_ld(A + row(REV ? t + 1 : t));
+        wx[i] = raw_ld(X + row(t));
+        if constexpr (REV) wh[i] = raw_ld(Hs + row(t - 1));
+    }
     float a[RUN], x[RUN];
 #pragma unroll
     for (int i = 0; i < RUN; ++i) {
-        const int p = p0 + i;
-        if (p < L) {
-            const int t = REV ? L - 1 - p : p;
-            if constexpr (REV)
-                a[i] = (t + 1 < L) ? ld(A + base + (int64_t)(t + 1) * ncols) : 0.f;
-            else
-                a[i] = (t > 0) ? ld(A + base + (int64_t)t * ncols) : 0.f;
-            x[i] = ld(X + base + (int64_t)t * ncols);
-        } else {
-            a[i] = 1.f;
-            x[i] = 0.f;
-        }
+        const bool has_a = p0 + i > 0 && p0 + i < L;  // A_0 (forward) and A_L (adjoint) do not enter
+        a[i] = has_a ? raw_f<T>(wa[i]) : 0.f;
+        x[i] = p0 + i < L ? raw_f<T>(wx[i]) : 0.f;
     }
     // the run's map h -> ra*h + rh
     float ra = 1.f, rh = 0.f;
@@ -175,7 +177,7 @@ __global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A
         if (p < L && cvalid) {
             const int t = REV ? L - 1 - p : p;
             st(Out + base + (int64_t)t * ncols, h);
-            if constexpr (REV) st(dAo + base + (int64_t)t * ncols, t > 0 ? h * ld(Hs + base + (int64_t)(t - 1) * ncols) : 0.f);
+            if constexpr (REV) st(dAo + base + (int64_t)t * ncols, t > 0 ? h * raw_f<T>(wh[i]) : 0.f);
         }
     }
 }

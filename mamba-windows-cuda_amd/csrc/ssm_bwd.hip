@@ -159,7 +159,7 @@ ssm_bwd_carry_kernel(const T* __restrict__ delta, const T* __restrict__ A, const
     constexpr bool XD = (XF & kXfDelta) != 0, XG = (XF & kXfGate) != 0;
     const T* zb = XG ? static_cast<const T*>(xf.z) : nullptr;
     const float lbias = XD && xf.delta_bias ? ld(static_cast<const T*>(xf.delta_bias) + ld_d) : 0.f;
-    T pd[SPG], py[SPG], pz[SPG], pc[BCPT];
+    raw_t<T> pd[SPG], py[SPG], pz[SPG], pc[BCPT];
     auto issue = [&](int k) {
         const int64_t ck = (int64_t)k * TC;
         const uint32_t rows = (uint32_t)min(TC, L - k * TC);
@@ -184,10 +184,10 @@ ssm_bwd_carry_kernel(const T* __restrict__ delta, const T* __restrict__ A, const
         float vmax = 0.f;
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
-            vd[s] = static_cast<float>(pd[s]);
-            vy[s] = static_cast<float>(py[s]);
+            vd[s] = raw_f<T>(pd[s]);
+            vy[s] = raw_f<T>(py[s]);
             if constexpr (XG) {  // the scan sees dout * silu(z)
-                const float zv = static_cast<float>(pz[s]);
+                const float zv = raw_f<T>(pz[s]);
                 vy[s] *= zv * sigmoid_f(zv);
             }
         }
@@ -215,7 +215,7 @@ ssm_bwd_carry_kernel(const T* __restrict__ delta, const T* __restrict__ A, const
 #pragma unroll
         for (int q = 0; q < BCPT; ++q) {
             const int e = tid * BCPT + q;
-            if (BCN >= 256 || e < BCN) s_c[buf][e / NS][e % NS] = static_cast<float>(pc[q]);
+            if (BCN >= 256 || e < BCN) s_c[buf][e / NS][e % NS] = raw_f<T>(pc[q]);
         }
     };
 
@@ -401,7 +401,7 @@ ssm_bwd_kernel(
     const int64_t rowD = row0 * D;
     constexpr bool XD = (XF & kXfDelta) != 0, XG = (XF & kXfGate) != 0;
     const T* zb = XG ? static_cast<const T*>(xf.z) : nullptr;
-    T pu[SPG], pd[SPG], py[SPG], pz[SPG], pyo[SPG], pb[BCPT], pc[BCPT];
+    raw_t<T> pu[SPG], pd[SPG], py[SPG], pz[SPG], pyo[SPG], pb[BCPT], pc[BCPT];
     float hnext[SPL];
     auto issue = [&](int k) {
         const int64_t ck = (int64_t)k * TC;
@@ -454,15 +454,15 @@ ssm_bwd_kernel(
         [[maybe_unused]] float vdz[SPG];
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
-            vd[s] = static_cast<float>(pd[s]);
-            vu[s] = static_cast<float>(pu[s]);
-            vy[s] = static_cast<float>(py[s]);
+            vd[s] = raw_f<T>(pd[s]);
+            vu[s] = raw_f<T>(pu[s]);
+            vy[s] = raw_f<T>(py[s]);
             if constexpr (XG) {  // out_z = out * silu(z): the scan sees dout * silu(z)
-                const float zv = static_cast<float>(pz[s]);
+                const float zv = raw_f<T>(pz[s]);
                 const float sz = sigmoid_f(zv);
                 const float a = vy[s] * sz;
                 // silu'(z) = sigmoid(z) * (1 + z * (1 - sigmoid(z)))
-                vdz[s] = a * static_cast<float>(pyo[s]) * __builtin_fmaf(zv, 1.f - sz, 1.f);
+                vdz[s] = a * raw_f<T>(pyo[s]) * __builtin_fmaf(zv, 1.f - sz, 1.f);
                 vy[s] = a * zv;
             }
         }
@@ -506,8 +506,8 @@ ssm_bwd_kernel(
             if (BCN >= 256 || e < BCN) {
                 const int n = e % NS;
                 float* row = &s_bc[e / NS][(n / SPL) * 2 * SPL + n % SPL];
-                row[0] = static_cast<float>(pb[q]);
-                row[SPL] = static_cast<float>(pc[q]);
+                row[0] = raw_f<T>(pb[q]);
+                row[SPL] = raw_f<T>(pc[q]);
             }
         }
     };

@@ -166,7 +166,7 @@ ssm_fwd_kernel(const T* __restrict__ u, const T* __restrict__ delta, const T* __
     // z is read only when the gated output is stored (the launcher sets kXfGate only with z and out_z)
     constexpr bool XD = (XF & kXfDelta) != 0, XG = HAS_OUT && (XF & kXfGate) != 0;
     const T* zb = XG ? static_cast<const T*>(xf.z) + row0 * D : nullptr;
-    T pu[SPG], pd[SPG], pz[SPG], pb[BCPT], pc[BCPT];
+    raw_t<T> pu[SPG], pd[SPG], pz[SPG], pb[BCPT], pc[BCPT];
     auto issue = [&](int k) {
         const int64_t ck = (int64_t)k * TC;
         const uint32_t rows = chunk_rows(k);
@@ -200,7 +200,7 @@ ssm_fwd_kernel(const T* __restrict__ u, const T* __restrict__ delta, const T* __
         float vd[SPG], vdu[SPG];
         float vmax = 0.f;
 #pragma unroll
-        for (int s = 0; s < SPG; ++s) vd[s] = static_cast<float>(pd[s]);
+        for (int s = 0; s < SPG; ++s) vd[s] = raw_f<T>(pd[s]);
         if constexpr (XD) {
 #pragma unroll
             for (int s = 0; s < SPG; ++s) vd[s] += lbias;  // 0 without a bias
@@ -218,11 +218,11 @@ ssm_fwd_kernel(const T* __restrict__ u, const T* __restrict__ delta, const T* __
         for (int s = 0; s < SPG; ++s) {
             vmax = __builtin_fmaxf(vmax, __builtin_fabsf(vd[s]));
             if constexpr (CARRY) sdt_l += vd[s];
-            const float vu = static_cast<float>(pu[s]);
+            const float vu = raw_f<T>(pu[s]);
             vdu[s] = vd[s] * vu;
             du_nxt[s] = Dl * vu;
             if constexpr (XG) {
-                const float zv = static_cast<float>(pz[s]);
+                const float zv = raw_f<T>(pz[s]);
                 gz_nxt[s] = zv * sigmoid_f(zv);  // silu(z)
             }
         }
@@ -236,10 +236,10 @@ ssm_fwd_kernel(const T* __restrict__ u, const T* __restrict__ delta, const T* __
                 const int n = e % NS;
                 if constexpr (HAS_OUT) {
                     float* row = &s_bc[buf][e / NS][(n / SPL) * 2 * SPL + n % SPL];
-                    row[0] = static_cast<float>(pb[q]);
-                    row[SPL] = static_cast<float>(pc[q]);
+                    row[0] = raw_f<T>(pb[q]);
+                    row[SPL] = raw_f<T>(pc[q]);
                 } else {
-                    s_bc[buf][e / NS][n] = static_cast<float>(pb[q]);
+                    s_bc[buf][e / NS][n] = raw_f<T>(pb[q]);
                 }
             }
         }
