@@ -191,6 +191,12 @@ int mwc_pscan_bwd(int dtype, const void* A, const void* H, const void* dH, void*
                   size_t workspace_bytes, void* stream);
 
 /*
+ * 1 if a scan of these sizes waits between tiles (bounded waits whose outcome the status functions below report),
+ * 0 if it has no wait that could give up, so its status is always MWC_OK. No reference counterpart.
+ */
+int mwc_pscan_waits(int64_t nseq, int64_t seqlen, int64_t ncols);
+
+/*
  * Outcome of the last mwc_pscan_fwd / mwc_pscan_bwd that used `workspace` with these sizes: waits
  * for `stream`, then returns MWC_OK, or MWC_ERR_INCOMPLETE if a bounded look-back wait between
  * tiles ran out (the affected outputs are then NaN, never a silently wrong value). No reference

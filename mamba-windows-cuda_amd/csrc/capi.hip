@@ -533,6 +533,10 @@ size_t mwc_pscan_workspace_size(int64_t nseq, int64_t seqlen, int64_t ncols) {
     return mwc::pscan_workspace_bytes(nseq, seqlen, ncols);
 }
 
+int mwc_pscan_waits(int64_t nseq, int64_t seqlen, int64_t ncols) {
+    return mwc::pscan_waits(nseq, seqlen, ncols) ? 1 : 0;
+}
+
 // Bound of each look-back wait of the scan (polls). MWC_PSCAN_SPIN_LIMIT overrides it (tests force a
 // give-up with 0: every wait then fails at once and every kernel still exits normally).
 static unsigned pscan_spin_limit() {

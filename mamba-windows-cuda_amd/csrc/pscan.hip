@@ -6,6 +6,9 @@
 // whose math is wrong for L >= 4): G_t = dH_t + A_{t+1}*G_{t+1}, dX = G,
 // dA_t = G_t*H_{t-1} for t >= 1 and dA_0 = 0.
 //
+// Two designs, chosen by use_chains: one wave per sequence (pscan_chain_kernel) for many narrow sequences, and the
+// tiled look-back scan described here.
+//
 // Design: one pass over HBM (12 B/element forward, 20 B/element backward).
 // A tile is TL consecutive steps x CW columns; each thread owns one column and
 // RUN consecutive steps held in VGPRs. Thread runs are combined inside the
@@ -182,10 +185,117 @@ __global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A
     }
 }
 
+// One wave per sequence of up to CW columns, for calls with sequences enough to fill the chip without
+// cutting L: the wave walks its sequence in tiles of (64/CW)*RUN steps with the state carried in a register, so
+// there are no tickets, flags, look-back or workgroup barriers. A lane owns one column and RUN consecutive steps
+// of a tile; the 64/CW runs of a column are joined by lane shuffles. The next tile's loads are in flight while a
+// tile is scanned. Bound: HBM.
+template <typename T, int CW, bool REV>
+__global__ void __launch_bounds__(kThreads) pscan_chain_kernel(const T* __restrict__ A, const T* __restrict__ X,
+                                                               const T* __restrict__ Hs, T* __restrict__ Out,
+                                                               T* __restrict__ dAo, unsigned* __restrict__ err, int L,
+                                                               int ncols, int64_t nseq) {
+    constexpr int R = 64 / CW;  // runs per tile
+    constexpr int RUN = sizeof(T) == 4 ? 8 : 16;  // steps per run: the same bytes in flight at 2 bytes an element
+    constexpr int TS = R * RUN;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // no wait that could give up
+    const int64_t seq = (int64_t)blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (seq >= nseq) return;
+    const int lane = threadIdx.x & 63;
+    const int col = lane % CW, r = lane / CW;
+    const int row_bytes = ncols * (int)sizeof(T);  // ncols <= 32: a tile's byte offsets are small
+    const int64_t base = seq * L * ncols;
+    const int ntile = (L + TS - 1) / TS;
+
+    // Tile n covers positions p = n*TS .. n*TS + TS - 1 in scan order: step t = p, or L - 1 - p for the adjoint.
+    // Rows are addressed from the tile's lowest step t0; offsets of positions at or past L (negative ones for the
+    // adjoint), of columns past ncols and of the neighbours that do not exist lie outside the resources, which
+    // return 0 for them and drop their stores.
+    auto first_row = [&](int n) { return REV ? max(0, L - (n + 1) * TS) : n * TS; };
+    auto lane_off = [&](int n, int i) {  // byte offset of the lane's step i from row first_row(n)
+        const int row = REV ? (L - 1 - n * TS - (r * RUN + i)) - first_row(n) : r * RUN + i;
+        return col < ncols ? (uint32_t)(row * row_bytes + col * (int)sizeof(T)) : kOob;
+    };
+    auto rsrc = [&](const T* p, int row) {  // rows [row, min(row + TS, L))
+        return make_rsrc(p + base + (int64_t)row * ncols, (uint32_t)(max(0, min(TS, L - row)) * row_bytes));
+    };
+    raw_t<T> na[RUN], nx[RUN], nh[REV ? RUN : 1];
+    auto issue = [&](int n) {
+        const int t0 = first_row(n);
+        // the adjoint's coefficient is A_{t+1} (none at t = L - 1) and its factor H_{t-1} (none at t = 0)
+        const rsrc_t ra = rsrc(A, REV ? t0 + 1 : t0), rx = rsrc(X, t0);
+        const int th = t0 > 0 ? t0 - 1 : 0;
+        const rsrc_t rh = rsrc(REV ? Hs : X, th);
+        const int dh = t0 > 0 ? 0 : row_bytes;
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            const uint32_t o = lane_off(n, i);
+            na[i] = buf_raw<T>(ra, o);
+            nx[i] = buf_raw<T>(rx, o);
+            if constexpr (REV) nh[i] = buf_raw<T>(rh, o - dh);
+        }
+    };
+    float h = 0.f;  // state entering the tile (the scan starts from 0)
+    issue(0);
+    for (int n = 0; n < ntile; ++n) {
+        float a[RUN], x[RUN], g[RUN];
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            a[i] = raw_f<T>(na[i]);
+            x[i] = raw_f<T>(nx[i]);
+            if constexpr (REV) g[i] = raw_f<T>(nh[i]);
+        }
+        if (!REV && n == 0) a[0] = r == 0 ? 0.f : a[0];  // A_0 is not used, whatever it holds
+        if (n + 1 < ntile) issue(n + 1);
+        float ra = 1.f, rh = 0.f;  // the run's map h -> ra*h + rh
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            rh = __builtin_fmaf(a[i], rh, x[i]);
+            ra *= a[i];
+        }
+        float s = h;  // state entering this lane's run; h becomes the one entering the next tile
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (q == r) s = h;
+            h = __builtin_fmaf(__shfl(ra, q * CW + col), h, __shfl(rh, q * CW + col));
+        }
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) x[i] = s = __builtin_fmaf(a[i], s, x[i]);
+        const int t0 = first_row(n);
+        const rsrc_t ro = rsrc(Out, t0), rd = rsrc(REV ? dAo : Out, t0);
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            const uint32_t o = lane_off(n, i);
+            buf_st<T>(ro, o, x[i]);
+            if constexpr (REV) {
+                float da = x[i] * g[i];
+                if (t0 == 0) da = L - 1 - n * TS - (r * RUN + i) == 0 ? 0.f : da;  // dA_0 = 0, whatever x holds
+                buf_st<T>(rd, o, da);
+            }
+        }
+    }
+}
+
+// Whether the one-wave-per-sequence kernel runs, at *cw columns a wave, rather than the tiled look-back kernel.
+// Forward and adjoint, against the look-back kernel: (768, 1024, 16) 45 and 83 us against 81 and 86 in fp32, 47 and
+// 83 against 79 and 81 in fp16; at (384, 1024, 16) too few bytes are in flight and the look-back kernel is as fast.
+// Sequences of up to 32 columns need more of them: (1024, 700, 32) fp16 64 and 120 us against 81 and 84, and
+// (2048, 300, 32) 36 and 67 against 79 and 82. Rows of 64 columns, whose look-back tiles hold four times a 16-column
+// one's bytes, stay there: (1024, 700, 64) fp16 87 and 107 us against 98 and 264 in waves of 64 columns.
+bool use_chains(int64_t nseq, int64_t ncols, int* cw) {
+    *cw = ncols <= 8 ? 8 : ncols <= 16 ? 16 : 32;
+    return ncols <= 32 && nseq >= (*cw == 32 ? 2048 : 768);
+}
+
 size_t pscan_workspace_bytes(int64_t nseq, int64_t seqlen, int64_t ncols) {
     if (nseq <= 0 || seqlen <= 0 || ncols <= 0) return 0;
     const PscanGeom g = geom(nseq, seqlen, ncols);
     return ((g.flag_bytes + 255) & ~(size_t)255) + 256;  // flags, then ticket + error word
+}
+
+bool pscan_waits(int64_t nseq, int64_t seqlen, int64_t ncols) {
+    int cw = 0;
+    return nseq > 0 && seqlen > 0 && ncols > 0 && !use_chains(nseq, ncols, &cw);
 }
 
 size_t pscan_error_word_offset(int64_t nseq, int64_t seqlen, int64_t ncols) {
@@ -202,9 +312,22 @@ static hipError_t pscan_t(const void* A, const void* X, const void* Hs, void* Ou
     unsigned* ticket = (unsigned*)((char*)ws + fb);
     unsigned* err = ticket + 1;
     const int64_t nwords = (int64_t)(fb + 256) / 8;
+    if (g.ntiles > INT32_MAX) return hipErrorInvalidValue;
+    int cw = 0;
+    if (use_chains(nseq, ncols, &cw)) {
+        const unsigned grid = (unsigned)((nseq + kThreads / 64 - 1) / (kThreads / 64));
+#define MWC_CHAIN_CW(CWV)                                                                                         \
+    if (cw == CWV)                                                                                                \
+        hipLaunchKernelGGL((pscan_chain_kernel<T, CWV, REV>), dim3(grid), dim3(kThreads), 0, st, (const T*)A,       \
+                           (const T*)X, (const T*)Hs, (T*)Out, (T*)dAo, err, (int)seqlen, (int)ncols, nseq);
+        MWC_CHAIN_CW(8)
+        MWC_CHAIN_CW(16)
+        MWC_CHAIN_CW(32)
+#undef MWC_CHAIN_CW
+        return hipGetLastError();
+    }
     const int cgrid = (int)std::min<int64_t>((nwords + 255) / 256, 4096);
     hipLaunchKernelGGL(pscan_clear_kernel, dim3(cgrid), dim3(256), 0, st, flags, nwords);
-    if (g.ntiles > INT32_MAX) return hipErrorInvalidValue;
 #define MWC_PSCAN_CW(CWV)                                                                                         \
     if (g.cw == CWV)                                                                                              \
         hipLaunchKernelGGL((pscan_kernel<T, CWV, REV>), dim3((unsigned)g.ntiles), dim3(kThreads), 0, st,          \

@@ -213,7 +213,8 @@ def pscan_forward(A, X):
         st = L_.mwc_pscan_fwd(_dtype_code(X), a3.data_ptr(), x3.data_ptr(), h3.data_ptr(), nseq, L, nc,
                               ws.data_ptr(), nbytes, _stream(X.device))
     _lib.check(st, "mwc_pscan_fwd")
-    _pscan_status(L_, ws, nbytes, nseq, L, nc, X.device, "mwc_pscan_fwd")
+    if L_.mwc_pscan_waits(nseq, L, nc):
+        _pscan_status(L_, ws, nbytes, nseq, L, nc, X.device, "mwc_pscan_fwd")
     return H
 
 
@@ -232,5 +233,6 @@ def pscan_backward(A, H, dH):
         st = L_.mwc_pscan_bwd(_dtype_code(H), a3.data_ptr(), h3.data_ptr(), g3.data_ptr(), da3.data_ptr(),
                               dx3.data_ptr(), nseq, L, nc, ws.data_ptr(), nbytes, _stream(H.device))
     _lib.check(st, "mwc_pscan_bwd")
-    _pscan_status(L_, ws, nbytes, nseq, L, nc, H.device, "mwc_pscan_bwd")
+    if L_.mwc_pscan_waits(nseq, L, nc):
+        _pscan_status(L_, ws, nbytes, nseq, L, nc, H.device, "mwc_pscan_bwd")
     return dA, dX

@@ -38,6 +38,31 @@ def test_pscan_forward_backward(dev, shape, dtype):
     np.testing.assert_allclose(_np(Ad.grad), rdA, **TOL[dtype])
 
 
+# Many narrow sequences run one wave each, in tiles of 64/CW runs (CW: 8, 16, 32 columns) of 8 fp32 or 16 16-bit
+# steps: the fewest sequences of each width and the shapes one below, lengths around a run and a tile.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(768, 1, 8), (769, 7, 3), (768, 9, 1), (768, 65, 8), (768, 129, 5), (770, 257, 8),
+                                   (768, 31, 16), (768, 33, 9), (767, 33, 16), (771, 64, 11), (768, 200, 16),
+                                   (2048, 17, 32), (2049, 33, 17), (2047, 33, 32), (2048, 100, 25)])
+def test_pscan_narrow_sequences(dev, shape, dtype):
+    print(f"case pscan narrow shape={shape} dtype={dtype}", flush=True)
+    g = torch.Generator().manual_seed(shape[0] + shape[1])
+    A = (0.5 + 0.5 * torch.rand(shape, generator=g)).to(dtype)
+    A[:, 0] = float("inf")  # A_0 is not used
+    X = torch.randn(shape, generator=g).to(dtype)
+    dH = torch.randn(shape, generator=g).to(dtype)
+    Ad, Xd = A.to(dev).requires_grad_(True), X.to(dev).requires_grad_(True)
+    H = parallel_scan_fn(Ad, Xd)
+    H.backward(dH.to(dev))
+    torch.cuda.synchronize()
+    A[:, 0] = 0
+    ref = orc.pscan_fwd(A, X)
+    rdA, rdX = orc.pscan_bwd(A, torch.from_numpy(ref), dH)
+    np.testing.assert_allclose(_np(H), ref, **TOL[dtype])
+    np.testing.assert_allclose(_np(Xd.grad), rdX, **TOL[dtype])
+    np.testing.assert_allclose(_np(Ad.grad), rdA, **TOL[dtype])
+
+
 def test_pscan_matches_reference_loop_and_ignores_A0(dev):
     """parallel_scan_ref semantics (pscan.py:153-171): H_0 = X_0 whatever A_0 is."""
     g = torch.Generator().manual_seed(2)
