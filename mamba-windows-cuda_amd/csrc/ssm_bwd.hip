@@ -129,6 +129,9 @@ ssm_bwd_carry_kernel(const T* __restrict__ delta, const T* __restrict__ A, const
     const int d0 = (wi.row % nblk_d) * CPB;
     const int k0 = first + seg * cps;
     const int k1 = min(nck, k0 + cps);
+    constexpr int AMS = LPC + 1;  // row stride of s_amax: it uses the staging buffer that the first chunk does not
+    static_assert(CPB * AMS <= 2 * CPB * RS, "s_amax fits a staging buffer");
+    float* const s_amax = &s_in[k1 & 1][0][0][0];
 
     const int wave = tid >> 6, lane = tid & 63;
     const int c = wave * CPW + lane / LPC;
@@ -148,9 +151,12 @@ ssm_bwd_carry_kernel(const T* __restrict__ delta, const T* __restrict__ A, const
         xs[j] = 0.f;  // the clamped exponents' departure from A2 * sum(delta)
     }
     float lamax2 = 0.f;  // max_n |A[ld_d][n]| * log2(e): the loader flags chunks that reach the clamp
+    {  // the lanes that hold the channel's states give it (as in the forward kernel)
+        float am = 0.f;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) lamax2 = __builtin_fmaxf(lamax2, __builtin_fabsf(ld(A + (int64_t)ld_d * NS + n)));
-    lamax2 *= kLog2e;
+        for (int j = 0; j < SPL; ++j) am = __builtin_fmaxf(am, __builtin_fabsf(A2[j]));
+        s_amax[c * AMS + lane % LPC] = am;
+    }
     float sdt_l = 0.f;  // the sum of the loader's delta values over the carry segment
 
     // buffer resources per chunk: rows past L and channels past D read as 0 (see the main kernel)
@@ -221,6 +227,8 @@ ssm_bwd_carry_kernel(const T* __restrict__ delta, const T* __restrict__ A, const
 
     if (tid < 2) s_flag[tid] = -1;
     __syncthreads();
+#pragma unroll
+    for (int q = 0; q < LPC; ++q) lamax2 = __builtin_fmaxf(lamax2, s_amax[lc * AMS + q]);
     if (k0 < k1) {
         issue(k1 - 1);
         commit(k1 - 1, (k1 - 1) & 1);
@@ -339,6 +347,9 @@ ssm_bwd_kernel(
     auto s_in = [&](int plane, int ch) -> float* { return &s_in_raw[plane * AS + ch * RS]; };
     __shared__ __align__(16) float s_part[4][TC][2 * NS];
     __shared__ __align__(16) float s_out[2][TC][OS];  // [du, ddelta][step][channel]
+    constexpr int AMS = LPC + 1;
+    static_assert(CPB * AMS <= 4 * 2 * PL, "s_amax fits the slabs");
+    float* const s_amax = &s_red[0][0];
     __shared__ int s_flag[2];  // [0]: index of the last staged chunk that needs the exponent clamp; [1]: sink
 
     const int tid = threadIdx.x;
@@ -435,9 +446,12 @@ ssm_bwd_kernel(
         ldv<SPL>(ckb + (int64_t)k * D * NS, hnext);
     };
     float lamax2 = 0.f;  // max_n |A[ld_d][n]| * log2(e): the loader flags chunks that reach the clamp
+    {  // the lanes that hold the channel's states give it (as in the forward kernel), through the fold's slabs
+        float am = 0.f;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) lamax2 = __builtin_fmaxf(lamax2, __builtin_fabsf(ld(A + (int64_t)ld_d * NS + n)));
-    lamax2 *= kLog2e;
+        for (int j = 0; j < SPL; ++j) am = __builtin_fmaxf(am, __builtin_fabsf(A2[j]));
+        s_amax[c * AMS + g] = am;
+    }
     const float lbias = XD && xf.delta_bias ? ld(static_cast<const T*>(xf.delta_bias) + ld_d) : 0.f;
     // d delta' / d delta (softplus) of the loader's elements, for the chunk being stored and the next
     float dd_cur[XD ? SPG : 1], dd_nxt[XD ? SPG : 1];
@@ -515,6 +529,8 @@ ssm_bwd_kernel(
     float hin[SPL];
     if (tid == 0) s_flag[0] = -1;
     __syncthreads();
+#pragma unroll
+    for (int q = 0; q < LPC; ++q) lamax2 = __builtin_fmaxf(lamax2, s_amax[lc * AMS + q]);
     if (k0 < k1) {  // L == 0 has no chunk; the outputs below are then dh_prev = dh_last and zero partials
         issue(k1 - 1);
         commit(k1 - 1);
