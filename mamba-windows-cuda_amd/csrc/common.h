@@ -65,12 +65,13 @@ template <typename T> __device__ __forceinline__ raw_t<T> raw_ld(const T* p) {
     else
         return *reinterpret_cast<const uint16_t*>(p);
 }
-template <typename T> __device__ __forceinline__ float raw_f(raw_t<T> v) {
+template <typename T> __device__ __forceinline__ T raw_v(raw_t<T> v) {
     if constexpr (sizeof(T) == 4)
         return v;
     else
-        return static_cast<float>(__builtin_bit_cast(T, (uint16_t)v));
+        return __builtin_bit_cast(T, (uint16_t)v);
 }
+template <typename T> __device__ __forceinline__ float raw_f(raw_t<T> v) { return static_cast<float>(raw_v<T>(v)); }
 template <typename T> __device__ __forceinline__ void buf_st(rsrc_t r, uint32_t off, float v);
 template <> __device__ __forceinline__ void buf_st<float>(rsrc_t r, uint32_t off, float v) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, off, 0, 0);
@@ -300,7 +301,7 @@ template <int G, int V> __device__ __forceinline__ float reduce_scatter(float (&
 // s_nop covers the read-after-VALU-write wait states of DPP and permlane sources.
 template <int CPW> constexpr int hi_log() { return CPW >= 16 ? 4 : CPW >= 8 ? 3 : CPW >= 4 ? 2 : CPW >= 2 ? 1 : 0; }
 template <int CPW> constexpr int hi_bit(int level) {
-    constexpr int order[6] = {4, 5, 3, 2, 1, 0};
+    constexpr int order[6] = {3, 2, 4, 5, 1, 0};
     int k = 0;
     for (int i = 0; i < 6; ++i)
         if (order[i] >= hi_log<CPW>()) {

@@ -412,7 +412,8 @@ ssm_bwd_kernel(
     const int64_t rowD = row0 * D;
     constexpr bool XD = (XF & kXfDelta) != 0, XG = (XF & kXfGate) != 0;
     const T* zb = XG ? static_cast<const T*>(xf.z) : nullptr;
-    raw_t<T> pu[SPG], pd[SPG], py[SPG], pz[SPG], pyo[SPG], pb[BCPT], pc[BCPT];
+    // held in the storage type: packed in pairs, 16-bit values leave registers that this kernel is short of
+    T pu[SPG], pd[SPG], py[SPG], pz[SPG], pyo[SPG], pb[BCPT], pc[BCPT];
     float hnext[SPL];
     auto issue = [&](int k) {
         const int64_t ck = (int64_t)k * TC;
@@ -422,17 +423,17 @@ ssm_bwd_kernel(
         const rsrc_t ry = make_rsrc(dout + rowD + ck * D, rows * row_bytes);
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
-            pu[s] = buf_raw<T>(ru, lofs + s * row_bytes);
-            pd[s] = buf_raw<T>(rd, lofs + s * row_bytes);
-            py[s] = buf_raw<T>(ry, lofs + s * row_bytes);
+            pu[s] = raw_v<T>(buf_raw<T>(ru, lofs + s * row_bytes));
+            pd[s] = raw_v<T>(buf_raw<T>(rd, lofs + s * row_bytes));
+            py[s] = raw_v<T>(buf_raw<T>(ry, lofs + s * row_bytes));
         }
         if constexpr (XG) {  // z and the ungated output, for dout * silu(z) and dz
             const rsrc_t rz = make_rsrc(zb + rowD + ck * D, rows * row_bytes);
             const rsrc_t ro = make_rsrc(yb_out + rowD + ck * D, rows * row_bytes);
 #pragma unroll
             for (int s = 0; s < SPG; ++s) {
-                pz[s] = buf_raw<T>(rz, lofs + s * row_bytes);
-                pyo[s] = buf_raw<T>(ro, lofs + s * row_bytes);
+                pz[s] = raw_v<T>(buf_raw<T>(rz, lofs + s * row_bytes));
+                pyo[s] = raw_v<T>(buf_raw<T>(ro, lofs + s * row_bytes));
             }
         }
         const uint32_t bc_bytes = rows * NS * sizeof(T);
@@ -440,8 +441,8 @@ ssm_bwd_kernel(
         const rsrc_t rc = make_rsrc(Cm + (row0 + ck) * NS, bc_bytes);
 #pragma unroll
         for (int q = 0; q < BCPT; ++q) {  // value e = tid*BCPT + q of the chunk's (step, n) rows
-            pb[q] = buf_raw<T>(rb, (tid * BCPT + q) * sizeof(T));
-            pc[q] = buf_raw<T>(rc, (tid * BCPT + q) * sizeof(T));
+            pb[q] = raw_v<T>(buf_raw<T>(rb, (tid * BCPT + q) * sizeof(T)));
+            pc[q] = raw_v<T>(buf_raw<T>(rc, (tid * BCPT + q) * sizeof(T)));
         }
         ldv<SPL>(ckb + (int64_t)k * D * NS, hnext);
     };
@@ -468,15 +469,15 @@ ssm_bwd_kernel(
         [[maybe_unused]] float vdz[SPG];
 #pragma unroll
         for (int s = 0; s < SPG; ++s) {
-            vd[s] = raw_f<T>(pd[s]);
-            vu[s] = raw_f<T>(pu[s]);
-            vy[s] = raw_f<T>(py[s]);
+            vd[s] = static_cast<float>(pd[s]);
+            vu[s] = static_cast<float>(pu[s]);
+            vy[s] = static_cast<float>(py[s]);
             if constexpr (XG) {  // out_z = out * silu(z): the scan sees dout * silu(z)
-                const float zv = raw_f<T>(pz[s]);
+                const float zv = static_cast<float>(pz[s]);
                 const float sz = sigmoid_f(zv);
                 const float a = vy[s] * sz;
                 // silu'(z) = sigmoid(z) * (1 + z * (1 - sigmoid(z)))
-                vdz[s] = a * raw_f<T>(pyo[s]) * __builtin_fmaf(zv, 1.f - sz, 1.f);
+                vdz[s] = a * static_cast<float>(pyo[s]) * __builtin_fmaf(zv, 1.f - sz, 1.f);
                 vy[s] = a * zv;
             }
         }
@@ -520,8 +521,8 @@ ssm_bwd_kernel(
             if (BCN >= 256 || e < BCN) {
                 const int n = e % NS;
                 float* row = &s_bc[e / NS][(n / SPL) * 2 * SPL + n % SPL];
-                row[0] = raw_f<T>(pb[q]);
-                row[SPL] = raw_f<T>(pc[q]);
+                row[0] = static_cast<float>(pb[q]);
+                row[SPL] = static_cast<float>(pc[q]);
             }
         }
     };
