@@ -447,11 +447,15 @@ ssm_bwd_kernel(
         ldv<SPL>(ckb + (int64_t)k * D * NS, hnext);
     };
     float lamax2 = 0.f;  // max_n |A[ld_d][n]| * log2(e): the loader flags chunks that reach the clamp
-    {  // the lanes that hold the channel's states give it (as in the forward kernel), through the fold's slabs
+    if constexpr (NS > 8) {  // the lanes that hold the channel's states give it (as in the forward kernel)
         float am = 0.f;
 #pragma unroll
         for (int j = 0; j < SPL; ++j) am = __builtin_fmaxf(am, __builtin_fabsf(A2[j]));
         s_amax[c * AMS + g] = am;
+    } else {  // few loads, and this instance spills at the register limit: 154 us against 167 (B=8 L=2048 D=1536)
+#pragma unroll
+        for (int n = 0; n < NS; ++n)
+            lamax2 = __builtin_fmaxf(lamax2, __builtin_fabsf(ld(A + (int64_t)ld_d * NS + n)) * kLog2e);
     }
     const float lbias = XD && xf.delta_bias ? ld(static_cast<const T*>(xf.delta_bias) + ld_d) : 0.f;
     // d delta' / d delta (softplus) of the loader's elements, for the chunk being stored and the next
@@ -530,8 +534,10 @@ ssm_bwd_kernel(
     float hin[SPL];
     if (tid == 0) s_flag[0] = -1;
     __syncthreads();
+    if constexpr (NS > 8) {
 #pragma unroll
-    for (int q = 0; q < LPC; ++q) lamax2 = __builtin_fmaxf(lamax2, s_amax[lc * AMS + q]);
+        for (int q = 0; q < LPC; ++q) lamax2 = __builtin_fmaxf(lamax2, s_amax[lc * AMS + q]);
+    }
     if (k0 < k1) {  // L == 0 has no chunk; the outputs below are then dh_prev = dh_last and zero partials
         issue(k1 - 1);
         commit(k1 - 1);
