@@ -253,7 +253,112 @@ SegPlan fill_plan(const SsmShape& s, bool bwd, int spl, int cap_main, int cap_ca
     return SegPlan{spl, 0, 0, 0, 0};
 }
 
-SegPlan plan_dir(const SsmShape& s, bool bwd) {
+// Small grids: modelled times in us. A pass costs its chunks at the rate of the waves that share a SIMD plus a
+// prologue for each round of workgroups, a carry pass its launch besides, and a main workgroup `fold` for each carry
+// that it folds into its start, one dependent load after the other; chunk times are those of a lone wave. Fitted to
+// every (states per lane, segments, carry split) measured at 31 shapes from (1, 256, 64) to (8, 2048, 1536) with N = 8,
+// 16, 32 and 64, in both directions. Its choice, where it is modelled at under 0.9 of the other rules' plan, is 4.9%
+// (forward) and 2.6% (backward) above the fastest plan of a shape on average against 13.5% and 8.8% without it; 0.95
+// made some shapes 2-4% slower. At 9 shapes it was not fitted to it gained 10% on average, (6, 400, 300) N=32 backward
+// 51 -> 36 us at best and (5, 100, 2000) 30.7 -> 32.3 at worst. The rules cut few channels too finely: they price
+// no fold, so (1, 1024, 256) fp32 ran 16 segments with carries split 4 ways, 19.9 and 28.4 us against 13.3 and 20.2.
+struct CostModel {
+    double fold, launch;
+    struct {
+        double main, carry;        // prologues
+        double rate[4], crate[4];  // relative rate of 2, 3, 4 and 6 or more waves per SIMD
+    } spl[3];                      // 1, 2 and 4 states per lane
+    struct {
+        double main, carry;  // one chunk of a lone wave
+    } chunk[4][3];           // by state count and states per lane; 0: not measured
+};
+const CostModel kFwdCost = {
+    0.135, 1.76,
+    {{3.80, 2.27, {1.44, 1.87, 2.14, 2.73}, {1.49, 1.66, 1.75, 2.02}},
+     {4.07, 2.65, {1.62, 2.17, 2.37, 2.47}, {1.02, 1.12, 1.19, 1.27}},
+     {9.47, 3.96, {1.49, 1.71, 1.91, 2.01}, {1.29, 1.32, 1.61, 1.71}}},
+    {{{0.69, 0.30}, {0.87, 0.54}, {0, 0}},
+     {{0.62, 0.37}, {0.86, 0.46}, {0, 0}},
+     {{0, 0}, {0.90, 0.44}, {1.32, 0.59}},
+     {{0, 0}, {0, 0}, {1.51, 0.53}}}};
+const CostModel kBwdCost = {
+    0.133, 3.77,
+    {{6.44, 1.88, {1.43, 1.78, 2.00, 2.10}, {1.38, 1.61, 1.77, 3.28}},
+     {5.69, 3.27, {1.47, 1.84, 2.04, 2.14}, {1.03, 1.20, 1.36, 1.50}},
+     {8.03, 6.51, {1.42, 1.72, 1.92, 2.02}, {1.68, 2.24, 4.26, 4.36}}},
+    {{{1.52, 0.28}, {2.13, 0.53}, {0, 0}},
+     {{1.50, 0.26}, {2.01, 0.46}, {0, 0}},
+     {{0, 0}, {2.04, 0.53}, {3.20, 0.93}},
+     {{0, 0}, {0, 0}, {4.13, 0.43}}}};
+
+double wave_rate(const double* r, int64_t q) {
+    return q <= 1 ? 1.0 : q >= 6 ? r[3] : q == 5 ? 0.5 * (r[2] + r[3]) : r[q - 2];
+}
+
+// pass_time with the model's costs
+double pass_us(int64_t wgs, int64_t chunks, int cap, double chunk, double prologue, const double* rate) {
+    if (wgs <= 0 || chunks <= 0) return 0.0;
+    const int64_t full = wgs / ((int64_t)kCUs * cap), rem = wgs - full * kCUs * cap;
+    double t = (double)full * ((double)chunks * chunk * cap / wave_rate(rate, cap) + prologue);
+    if (rem > 0) {
+        const int64_t q = (rem + kCUs - 1) / kCUs;
+        t += (double)chunks * chunk * q / wave_rate(rate, q) + prologue;
+    }
+    return t;
+}
+
+double plan_us(const SsmShape& s, bool bwd, const SegPlan& p, int cap_main, int cap_carry) {
+    const CostModel& m = bwd ? kBwdCost : kFwdCost;
+    const int ni = s.nstate == 8 ? 0 : s.nstate == 16 ? 1 : s.nstate == 32 ? 2 : 3, si = p.spl == 4 ? 2 : p.spl - 1;
+    const auto& c = m.chunk[ni][si];
+    const int64_t w1 = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl));
+    double t = pass_us(w1 * p.nseg, p.cps, cap_main, c.main, m.spl[si].main, m.spl[si].rate);
+    if (p.nseg > 1)
+        t += m.launch + pass_us(w1 * p.ncar, p.cps / p.cfold, cap_carry, c.carry, m.spl[si].carry, m.spl[si].crate) +
+             m.fold * (bwd ? p.ncar : (p.nseg - 1) * p.cfold);
+    return t;
+}
+
+// The model's plan where it undercuts `p` clearly, else `p`. Never one whose carries need more scratch than `p`'s and
+// than the scratch of mwc_ssm_fwd_noalloc, so that no size which that entry point takes gets refused.
+SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
+    const int64_t nck = (s.seqlen + kCkptSteps - 1) / kCkptSteps;
+    const int64_t w1 = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl));
+    const int ni = s.nstate == 8 ? 0 : s.nstate == 16 ? 1 : s.nstate == 32 ? 2 : 3;
+    if (w1 <= 0 || nck < 2 || w1 >= (int64_t)kCUs * 3 / 2 || kFwdCost.chunk[ni][p.spl == 4 ? 2 : p.spl - 1].main == 0)
+        return p;
+    auto caps = [&](int spl, int& cm, int& cc) {
+        cm = bwd ? bwd_cap(s.nstate, spl) : fwd_cap(s.nstate, spl);
+        cc = bwd ? bwd_carry_cap(s.nstate, spl) : fwd_carry_cap(s.nstate, spl);
+    };
+    int cm = 0, cc = 0;
+    caps(p.spl, cm, cc);
+    SegPlan best = p;
+    double best_t = 0.9 * plan_us(s, bwd, p, cm, cc);
+    const size_t most = std::max<size_t>(carry_bytes(s, p), MWC_NOALLOC_SCRATCH_BYTES / 2);
+    for (int spl = 1; spl <= 4; spl *= 2) {
+        if (kFwdCost.chunk[ni][spl == 4 ? 2 : spl - 1].main == 0) continue;
+        caps(spl, cm, cc);
+        const int64_t ws = s.batch * ((s.dim + cpb_of(s.nstate, spl) - 1) / cpb_of(s.nstate, spl));
+        for (int n : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48}) {
+            for (int f = 1; f <= (n > 1 ? 4 : 1); f *= 2) {
+                const int64_t cps = ((nck + n - 1) / n + f - 1) / f * f, nseg = (nck + cps - 1) / cps, ccps = cps / f;
+                if (n > 1 && nseg < 2) continue;
+                const int64_t ncar = nseg < 2 ? 0 : bwd ? (nck - cps + ccps - 1) / ccps : (nseg - 1) * f;
+                const SegPlan q{spl, (int)nseg, (int)cps, f, (int)ncar};
+                if (ws * nseg > INT32_MAX / 2 || carry_bytes(s, q) > most) continue;
+                const double t = plan_us(s, bwd, q, cm, cc);
+                if (t < best_t) {
+                    best_t = t;
+                    best = q;
+                }
+            }
+        }
+    }
+    return best;
+}
+
+SegPlan plan_rules(const SsmShape& s, bool bwd) {
     auto caps = [&](int spl, int& cm, int& cc) {
         cm = bwd ? bwd_cap(s.nstate, spl) : fwd_cap(s.nstate, spl);
         cc = bwd ? bwd_carry_cap(s.nstate, spl) : fwd_carry_cap(s.nstate, spl);
@@ -279,6 +384,24 @@ SegPlan plan_dir(const SsmShape& s, bool bwd) {
     if (p.nseg > 1 && x_forced < 0 && rows < (int64_t)kCUs * cm) return p;
     const SegPlan h = split_plan(s, bwd, spl, cm, cc, rel, x_forced, &th);
     return h.nseg > 0 && (x_forced > 0 || th < t * 0.98) ? h : p;
+}
+
+// The plan of the last shape that this thread asked for is kept, per direction: a call asks for it three times, and a
+// loop for the same shape each time. Overrides (tuning and tests) are read on every call.
+SegPlan plan_dir(const SsmShape& s, bool bwd) {
+    for (const char* e : {"MWC_SPL", "MWC_NSEG", "MWC_CFOLD", "MWC_NSPLIT"})
+        if (getenv(e) != nullptr) return plan_rules(s, bwd);
+    static thread_local struct {
+        SsmShape s{-1, -1, -1, 0};
+        SegPlan p;
+    } last[2];
+    auto& l = last[bwd];
+    if (l.s.batch != s.batch || l.s.seqlen != s.seqlen || l.s.dim != s.dim || l.s.nstate != s.nstate) {
+        const SegPlan p = plan_rules(s, bwd);
+        l.p = p.nfull > 0 ? p : small_grid_plan(s, bwd, p);
+        l.s = s;
+    }
+    return l.p;
 }
 
 }  // namespace

@@ -189,6 +189,26 @@ def test_planner_partly_split_rounds(dev, monkeypatch, idx):
     _run_case(dev, monkeypatch, 30000 + idx, conditioned=False, c=c)
 
 
+# Small grids, where the planner chooses by modelled time: unsplit, many short segments, a single chunk in the last
+# segment, each state count. (The gradients' bound is the conditioned one: they sum over up to 2048 steps.)
+SMALL_CASES = [dict(B=1, L=1024, D=256, n=16, dtype=torch.float32, seed=601),
+               dict(B=2, L=777, D=333, n=16, dtype=torch.bfloat16, seed=602),
+               dict(B=1, L=64, D=2560, n=16, dtype=torch.float16, seed=603),
+               dict(B=1, L=17, D=40, n=8, dtype=torch.float32, seed=604),
+               dict(B=2, L=1009, D=100, n=8, dtype=torch.float16, seed=605),
+               dict(B=6, L=400, D=300, n=32, dtype=torch.float16, seed=606),
+               dict(B=2, L=200, D=64, n=64, dtype=torch.float32, seed=607)]
+
+
+@pytest.mark.parametrize("idx", range(len(SMALL_CASES)))
+def test_planner_small_grids(dev, monkeypatch, idx):
+    c = dict(with_h=True, bias=False, softplus=False, gate=False, spl=None, nseg=None, cfold=None, lvl=idx % 2,
+             **SMALL_CASES[idx])
+    for var in ("MWC_SPL", "MWC_NSEG", "MWC_CFOLD", "MWC_NSPLIT"):
+        monkeypatch.delenv(var, raising=False)
+    _run_case(dev, monkeypatch, 40000 + idx, conditioned=True, c=c)
+
+
 @pytest.mark.parametrize("idx", CONDITIONED)
 def test_conditioned_case(dev, monkeypatch, idx):
     _run_case(dev, monkeypatch, idx, conditioned=True)
