@@ -257,10 +257,10 @@ SegPlan fill_plan(const SsmShape& s, bool bwd, int spl, int cap_main, int cap_ca
 // prologue for each round of workgroups, a carry pass its launch besides, and a main workgroup `fold` for each carry
 // that it folds into its start, one dependent load after the other; chunk times are those of a lone wave. Fitted to
 // every (states per lane, segments, carry split) measured at 31 shapes from (1, 256, 64) to (8, 2048, 1536) with N = 8,
-// 16, 32 and 64, in both directions. Its choice, where it is modelled at under 0.9 of the other rules' plan, is 4.9%
-// (forward) and 2.6% (backward) above the fastest plan of a shape on average against 13.5% and 8.8% without it; 0.95
-// made some shapes 2-4% slower. At 9 shapes it was not fitted to it gained 10% on average, (6, 400, 300) N=32 backward
-// 51 -> 36 us at best and (5, 100, 2000) 30.7 -> 32.3 at worst. The rules cut few channels too finely: they price
+// 16, 32 and 64, in both directions. Its choice, where it is modelled at under 0.9 (backward 0.95) of the other rules'
+// plan, is 4.9% (forward) and 2.1% (backward) above the fastest plan of a shape on average against 13.5% and 8.8%
+// without it; at 0.95 some forwards got 2-4% slower. At 9 shapes it was not fitted to it gained 10% on average,
+// (6, 400, 300) N=32 backward 51 -> 36 us at best and (5, 100, 2000) 30.7 -> 32.3 at worst. The rules cut few channels too finely: they price
 // no fold, so (1, 1024, 256) fp32 ran 16 segments with carries split 4 ways, 19.9 and 28.4 us against 13.3 and 20.2.
 struct CostModel {
     double fold, launch;
@@ -334,7 +334,7 @@ SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
     int cm = 0, cc = 0;
     caps(p.spl, cm, cc);
     SegPlan best = p;
-    double best_t = 0.9 * plan_us(s, bwd, p, cm, cc);
+    double best_t = (bwd ? 0.95 : 0.9) * plan_us(s, bwd, p, cm, cc);
     const size_t most = std::max<size_t>(carry_bytes(s, p), MWC_NOALLOC_SCRATCH_BYTES / 2);
     for (int spl = 1; spl <= 4; spl *= 2) {
         if (kFwdCost.chunk[ni][spl == 4 ? 2 : spl - 1].main == 0) continue;
@@ -343,11 +343,12 @@ SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
         for (int n : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48}) {
             for (int f = 1; f <= (n > 1 ? 4 : 1); f *= 2) {
                 const int64_t cps = ((nck + n - 1) / n + f - 1) / f * f, nseg = (nck + cps - 1) / cps, ccps = cps / f;
-                if (n > 1 && nseg < 2) continue;
+                if (n > 1 && (nseg < 2 || cps < 2)) continue;  // segments of one chunk run longer than modelled
                 const int64_t ncar = nseg < 2 ? 0 : bwd ? (nck - cps + ccps - 1) / ccps : (nseg - 1) * f;
                 const SegPlan q{spl, (int)nseg, (int)cps, f, (int)ncar};
                 if (ws * nseg > INT32_MAX / 2 || carry_bytes(s, q) > most) continue;
-                const double t = plan_us(s, bwd, q, cm, cc);
+                double t = plan_us(s, bwd, q, cm, cc);
+                if (bwd && nseg < 2) t *= 0.95 / 0.9;  // so do unsplit backwards
                 if (t < best_t) {
                     best_t = t;
                     best = q;
