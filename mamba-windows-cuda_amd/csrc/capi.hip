@@ -719,8 +719,7 @@ int mwc_pscan_status(const void* workspace, size_t workspace_bytes, int64_t nseq
         return fail(MWC_ERR_WORKSPACE, "scan workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
     unsigned err = 0;
     hipStream_t st = (hipStream_t)stream;
-    MWC_HIP_TRY(hipMemcpyAsync(&err, (const char*)workspace + mwc::pscan_error_word_offset(nseq, seqlen, ncols),
-                               sizeof(err), hipMemcpyDeviceToHost, st));
+    MWC_HIP_TRY(hipMemcpyAsync(&err, workspace, sizeof(err), hipMemcpyDeviceToHost, st));  // its first word
     MWC_HIP_TRY(hipStreamSynchronize(st));
     if (err != 0)
         return fail(MWC_ERR_INCOMPLETE,
@@ -739,8 +738,7 @@ int mwc_pscan_status_async(const void* workspace, size_t workspace_bytes, int64_
     const size_t need = mwc::pscan_workspace_bytes(nseq, seqlen, ncols);
     if (workspace == nullptr || workspace_bytes < need)
         return fail(MWC_ERR_WORKSPACE, "scan workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
-    MWC_HIP_TRY(hipMemcpyAsync(host_word, (const char*)workspace + mwc::pscan_error_word_offset(nseq, seqlen, ncols),
-                               sizeof(uint32_t), hipMemcpyDeviceToHost, (hipStream_t)stream));
+    MWC_HIP_TRY(hipMemcpyAsync(host_word, workspace, sizeof(uint32_t), hipMemcpyDeviceToHost, (hipStream_t)stream));
     return MWC_OK;
 }
 

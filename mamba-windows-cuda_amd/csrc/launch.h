@@ -150,10 +150,8 @@ hipError_t launch_pscan_fwd(int dt, const void* A, const void* X, void* H, int64
 hipError_t launch_pscan_bwd(int dt, const void* A, const void* H, const void* dH, void* dA,
                             void* dX, int64_t nseq, int64_t seqlen, int64_t ncols, void* ws,
                             unsigned spin_limit, hipStream_t st);
-size_t pscan_workspace_bytes(int64_t nseq, int64_t seqlen, int64_t ncols);
-size_t pscan_error_word_offset(int64_t nseq, int64_t seqlen, int64_t ncols);  // byte offset in the workspace
-// Whether the scan of these sizes waits on look-back flags (and so can give up), rather than walking each sequence
-// in one wave.
+size_t pscan_workspace_bytes(int64_t nseq, int64_t seqlen, int64_t ncols);  // its first word is the error word
+// Whether the scan of these sizes waits on look-back flags (and so can give up): not with one tile along L.
 bool pscan_waits(int64_t nseq, int64_t seqlen, int64_t ncols);
 constexpr unsigned kPscanSpinLimit = 1u << 22;  // default bound of a look-back wait (polls of ~128 clocks)
 

@@ -38,12 +38,13 @@ def test_pscan_forward_backward(dev, shape, dtype):
     np.testing.assert_allclose(_np(Ad.grad), rdA, **TOL[dtype])
 
 
-# Many narrow sequences run one wave each, in tiles of 64/CW runs (CW: 8, 16, 32 columns) of 8 fp32 or 16 16-bit
-# steps: the fewest sequences of each width and the shapes one below, lengths around a run and a tile.
+# Narrow sequences run in tiles of 8 or 16 columns by 256 steps and 32 columns by 128, the columns of one lane each;
+# a single tile along L has no look-back. Lengths around a run, a tile and two.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shape", [(768, 1, 8), (769, 7, 3), (768, 9, 1), (768, 65, 8), (768, 129, 5), (770, 257, 8),
                                    (768, 31, 16), (768, 33, 9), (767, 33, 16), (771, 64, 11), (768, 200, 16),
-                                   (2048, 17, 32), (2049, 33, 17), (2047, 33, 32), (2048, 100, 25)])
+                                   (2048, 17, 32), (2049, 33, 17), (2047, 33, 32), (2048, 100, 25),
+                                   (5, 513, 8), (3, 256, 16), (9, 1025, 10), (4, 129, 32)])
 def test_pscan_narrow_sequences(dev, shape, dtype):
     print(f"case pscan narrow shape={shape} dtype={dtype}", flush=True)
     g = torch.Generator().manual_seed(shape[0] + shape[1])
@@ -56,6 +57,34 @@ def test_pscan_narrow_sequences(dev, shape, dtype):
     H.backward(dH.to(dev))
     torch.cuda.synchronize()
     A[:, 0] = 0
+    ref = orc.pscan_fwd(A, X)
+    rdA, rdX = orc.pscan_bwd(A, torch.from_numpy(ref), dH)
+    np.testing.assert_allclose(_np(H), ref, **TOL[dtype])
+    np.testing.assert_allclose(_np(Xd.grad), rdX, **TOL[dtype])
+    np.testing.assert_allclose(_np(Ad.grad), rdA, **TOL[dtype])
+
+
+# Pairs of 16-bit columns: 33 to 64 and more, whole and ragged column blocks, and the odd widths, fewer tiles and
+# misaligned tensors that stay with single columns. The 68 column blocks
+# of 17 tiles share tickets in groups of 34, the 65 in groups of 33 and 32.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,offset", [((128, 5, 34), 0), ((130, 128, 64), 0), ((64, 130, 66), 0), ((64, 257, 62), 1),
+                                          ((3, 2049, 382), 0), ((3, 2049, 382), 1), ((3, 2049, 381), 0),
+                                          ((2, 300, 1050), 0), ((4, 2100, 1050), 0), ((65, 2100, 64), 1), ((1, 129, 130), 0)])
+def test_pscan_column_pairs(dev, shape, offset, dtype):
+    print(f"case pscan pairs shape={shape} offset={offset} dtype={dtype}", flush=True)
+    g = torch.Generator().manual_seed(shape[0] + shape[1])
+    A = (0.5 + 0.5 * torch.rand(shape, generator=g)).to(dtype)
+    X, dH = (torch.randn(shape, generator=g).to(dtype) for _ in range(2))
+
+    def put(t):  # contiguous, `offset` elements into its storage
+        s = torch.empty(t.numel() + offset, dtype=dtype, device=dev)[offset:].view(shape)
+        return s.copy_(t.to(dev)).requires_grad_(True)
+
+    Ad, Xd = put(A), put(X)
+    H = parallel_scan_fn(Ad, Xd)
+    H.backward(dH.to(dev))
+    torch.cuda.synchronize()
     ref = orc.pscan_fwd(A, X)
     rdA, rdX = orc.pscan_bwd(A, torch.from_numpy(ref), dH)
     np.testing.assert_allclose(_np(H), ref, **TOL[dtype])
