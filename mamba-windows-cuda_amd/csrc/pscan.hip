@@ -15,9 +15,8 @@
 // a single relaxed agent-scope atomic carries both the flag and the value
 // (no cache-wide release/acquire fences). Tiles are taken from an atomic
 // ticket (see ticket_chains), so every predecessor of a waiting tile is
-// already resident, and each
-// spin is bounded so a lost update can never hang the device. A wait that runs
-// out of spins sets the workspace's error word (read by mwc_pscan_status) and
+// already resident, and each spin is bounded so a lost update can never hang
+// the device. A wait that runs out of spins sets the workspace's error word (read by mwc_pscan_status) and
 // gives the tile a NaN prefix, so its outputs, and every later tile's, are NaN
 // rather than a plausible wrong value.
 #include <algorithm>
