@@ -19,6 +19,13 @@
 // the device. A wait that runs out of spins sets the workspace's error word (read by mwc_pscan_status) and
 // gives the tile a NaN prefix, so its outputs, and every later tile's, are NaN
 // rather than a plausible wrong value.
+//
+// Range: the coefficient of a map over many steps is a product that leaves fp32 long before the states do (1.42^256
+// overflows, 0.66^256 is 0), and inf * 0 is NaN. So such products carry an exponent of their own, from a thread's run
+// to the look-back: states of 0, tiny ones and infinite ones pass through any number of finite coefficients as they do
+// step by step. Where no product leaves fp32 the results are the same bit for bit; the checks cost up to 2% in fp32 and
+// 6% in 16 bits ((2048, 300, 32) fp16 27.1 -> 28.7 us), exponents in every tile up to 12% ((1, 30000, 16) fp16 14.5 ->
+// 16.3); calls of 64 columns and more are unchanged.
 #include <algorithm>
 
 #include "common.h"
@@ -80,6 +87,19 @@ __device__ __forceinline__ uint64_t pack(uint32_t st, float v) {
     return ((uint64_t)st << 32) | (uint64_t)__builtin_bit_cast(uint32_t, v);
 }
 __device__ __forceinline__ float unpack_v(uint64_t w) { return __builtin_bit_cast(float, (uint32_t)(w & 0xffffffffu)); }
+// A tile's coefficient m * 2^e: e above the two status bits (at most 256 steps of |e| <= 149, so it fits 30 bits).
+__device__ __forceinline__ uint64_t pack_coef(uint32_t st, float m, int e) { return pack(st | (uint32_t)e << 2, m); }
+__device__ __forceinline__ int unpack_e(uint64_t w) { return (int)(uint32_t)(w >> 32) >> 2; }
+
+// Whether a product is not safely inside fp32's normal range (NaN included)
+__device__ __forceinline__ bool out_of_range(float m) {
+    m = __builtin_fabsf(m);
+    return !(m >= 0x1p-100f && m <= 0x1p100f);
+}
+// m * 2^e * h + b, rounded once where h * 2^e is a normal number
+__device__ __forceinline__ float apply(float m, int e, float h, float b) {
+    return __builtin_fmaf(m, __builtin_ldexpf(h, e), b);
+}
 
 __device__ __forceinline__ void publish(uint64_t* p, uint64_t w) {
     __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -128,9 +148,10 @@ template <typename T, int V> __device__ __forceinline__ void row_st(T* p, const 
 
 // REV = false: forward scan of X with coefficients A (A_0 ignored) into Out.
 // REV = true : adjoint; X = dH, Out = dX, Hs = forward H, dAo = dA.
-// A thread owns V adjacent columns (2: 16-bit pairs).
+// A thread owns V adjacent columns (2: 16-bit pairs). Waves: 80 VGPRs leave 6 a SIMD, which the exponents' code would
+// exceed by two registers; the adjoint's 16 more values fit 5.
 template <typename T, int CW, int V, bool REV>
-__global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A, const T* __restrict__ X,
+__global__ void __launch_bounds__(kThreads, CW == 64 ? 3 : CW == 8 ? 8 : REV ? 5 : 6) pscan_kernel(const T* __restrict__ A, const T* __restrict__ X,
                                                          const T* __restrict__ Hs, T* __restrict__ Out,
                                                          T* __restrict__ dAo, uint64_t* __restrict__ flags,
                                                          unsigned* __restrict__ tickets, unsigned* __restrict__ err,
@@ -138,16 +159,19 @@ __global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A
                                                          unsigned ngroups, unsigned spin_limit) {
     constexpr int R = kThreads / CW;     // thread rows per tile
     constexpr int TS = tile_steps(CW), RUN = TS / R;  // steps of a tile and of a thread
-    __shared__ int s_tile;
+    __shared__ int s_tile, s_wide;
     __shared__ float s_a[R][V][CW], s_h[R][V][CW], s_p[V][CW];
+    __shared__ int s_e[R][V][CW];  // exponents of s_a, read where s_wide: some run's coefficient leaves fp32
 
     // a ticket group's tiles: its column blocks, all at one step range before the next
     const unsigned group = blockIdx.x % ngroups;
     const int64_t chain0 = (int64_t)group * gchains;
     const int gw = (int)min((int64_t)gchains, nchains - chain0);
     const int nltile = (L + TS - 1) / TS;
-    if (threadIdx.x == 0)  // one tile along L: nothing waits, so any order does
+    if (threadIdx.x == 0) {  // one tile along L: nothing waits, so any order does
         s_tile = nltile > 1 ? (int)atomicAdd(tickets + (size_t)group * kTicketStride, 1u) : (int)(blockIdx.x / ngroups);
+        s_wide = 0;
+    }
     if (nltile == 1 && blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // nor is the workspace cleared
     __syncthreads();
     const int lt = s_tile / gw;  // position of the tile along L (in scan order)
@@ -184,42 +208,73 @@ __global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A
         float ra = 1.f, rh = 0.f;
 #pragma unroll
         for (int i = 0; i < RUN; ++i) {
+            if constexpr (V == 2) asm volatile("" : "+v"(wa[i]), "+v"(wx[i]));  // see the second pass below
             const float a = row_val<T>(wa[i], v);
             rh = __builtin_fmaf(a, rh, row_val<T>(wx[i], v));
             ra *= a;
         }
+        // Out of this range the product is formed again from mantissas and exponents (rare: one compare a run). The
+        // first run's coefficient has no state to multiply, and that of a run past the end is not used.
+        int re = 0;
+        if (out_of_range(ra) && p0 > 0 && p0 + RUN <= L) {
+            ra = 1.f;
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) {
+                const float p = ra * row_val<T>(wa[i], v);
+                re += __builtin_amdgcn_frexp_expf(p);
+                ra = __builtin_amdgcn_frexp_mantf(p);
+            }
+            s_wide = 1;
+        }
         s_a[r][v][cl] = ra;
+        s_e[r][v][cl] = re;
         s_h[r][v][cl] = rh;
     }
     __syncthreads();
 
+    const bool wide = s_wide != 0;
     if (r < V) {  // thread row v joins the tiles' column v of each thread
-        float ta = 1.f, th = 0.f;  // the tile's map
+        float ta = 1.f, th = 0.f;  // the tile's map ta * 2^te * h + th
+        int te = 0;
 #pragma unroll
         for (int q = 0; q < R; ++q) {
             th = __builtin_fmaf(s_a[q][r][cl], th, s_h[q][r][cl]);
             ta *= s_a[q][r][cl];
+        }
+        if (wide || (lt > 0 && out_of_range(ta))) {  // again with exponents: a product of R mantissas is above 2^-R
+            ta = 1.f, th = 0.f;
+#pragma unroll 2  // all at once the loads take 30 to 60 registers more, and the waves that they hold
+            for (int q = 0; q < R; ++q) {
+                const float qa = s_a[q][r][cl];
+                const int qe = s_e[q][r][cl];
+                th = apply(qa, qe, th, s_h[q][r][cl]);
+                ta *= __builtin_amdgcn_frexp_mantf(qa);
+                te += qe + __builtin_amdgcn_frexp_expf(qa);
+            }
         }
         uint64_t* f = flags + ((chain * nltile + lt) * (CW * V) + r * CW + cl) * 2;
         float prefix = 0.f;  // state entering the tile (the scan starts from 0; t = 0 ignores A_0)
         if (lt == 0) {
             if (nltile > 1) publish(f, pack(kStInc, th));
         } else {
-            publish(f + 1, pack(kStAgg, ta));
+            publish(f + 1, pack_coef(kStAgg, ta, te));
             publish(f, pack(kStAgg, th));
             float acc_a = 1.f, acc_h = 0.f;  // map of the tiles between the predecessor and this one
+            int acc_e = 0;
             uint64_t* pf = f - (int64_t)(CW * V) * 2;
             for (int j = lt - 1; j >= 0; --j, pf -= (int64_t)(CW * V) * 2) {
                 const uint64_t w = wait_word(pf, err, spin_limit);
                 if ((w >> 32) == kStInc) {
-                    prefix = __builtin_fmaf(acc_a, unpack_v(w), acc_h);
+                    prefix = apply(acc_a, acc_e, unpack_v(w), acc_h);
                     break;
                 }
                 const uint64_t wa = wait_word(pf + 1, err, spin_limit);
-                acc_h = __builtin_fmaf(acc_a, unpack_v(w), acc_h);
+                acc_h = apply(acc_a, acc_e, unpack_v(w), acc_h);
                 acc_a *= unpack_v(wa);
+                acc_e += unpack_e(wa) + __builtin_amdgcn_frexp_expf(acc_a);
+                acc_a = __builtin_amdgcn_frexp_mantf(acc_a);
             }
-            publish(f, pack(kStInc, __builtin_fmaf(ta, prefix, th)));
+            publish(f, pack(kStInc, apply(ta, te, prefix, th)));
         }
         s_p[r][cl] = prefix;
     }
@@ -230,7 +285,11 @@ __global__ void __launch_bounds__(kThreads) pscan_kernel(const T* __restrict__ A
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         h[v] = s_p[v][cl];
-        for (int q = 0; q < r; ++q) h[v] = __builtin_fmaf(s_a[q][v][cl], h[v], s_h[q][v][cl]);
+        if (wide)
+#pragma unroll 1
+            for (int q = 0; q < r; ++q) h[v] = apply(s_a[q][v][cl], s_e[q][v][cl], h[v], s_h[q][v][cl]);
+        else
+            for (int q = 0; q < r; ++q) h[v] = __builtin_fmaf(s_a[q][v][cl], h[v], s_h[q][v][cl]);
     }
 #pragma unroll
     for (int i = 0; i < RUN; ++i) {

@@ -92,6 +92,57 @@ def test_pscan_column_pairs(dev, shape, offset, dtype):
     np.testing.assert_allclose(_np(Ad.grad), rdA, **TOL[dtype])
 
 
+def _range_inputs(kind, a, shape, dtype):
+    """Sequences whose coefficients multiply out of fp32's range over a run, a tile or two while the scan itself stays
+    in it. zero: nothing enters before the scan's last 20 steps (the adjoint's: before its first 20). tiny: 1e-30
+    enters first, and grows. inf: an infinity enters early and stays, whatever the decay."""
+    L = shape[1]
+    g = torch.Generator().manual_seed(L + shape[2])
+    A = torch.full(shape, a)
+    X, dH = torch.zeros(shape), torch.zeros(shape)
+    if kind == "zero":
+        A[:, :24] = A[:, -24:] = 0.5
+        X[:, -20:] = torch.randn(shape[0], 20, shape[2], generator=g)
+        dH[:, :20] = torch.randn(shape[0], 20, shape[2], generator=g)
+    elif kind == "tiny":  # up to 1e-30 * a^n <= 1e15, from the start of a run on
+        n = int(np.log(1e45) / np.log(abs(a)))
+        lo = L // 64 * 32
+        A[:, :lo] = 1.0
+        A[:, lo + n:] = 1.0
+        X[:, 0] = dH[:, -1] = 1e-30
+    else:
+        X[:, 10, ::2] = float("inf")
+        X[:, 10, 1::2] = -float("inf")
+        dH[:, -10] = X[:, 10]
+        X[:, 3] = 1.0
+    return A.to(dtype), X.to(dtype), dH.to(dtype)
+
+
+# Narrow and wide tiles, pairs (128 columns in 16 bits), several tiles along L and one; mean coefficients that leave
+# fp32 over 2 tiles (1.3), one (1.5, 3), a run of 16 or 32 steps (300; 0.01 downwards).
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(3, 1024, 8), (2, 1100, 16), (3, 1024, 32), (2, 1024, 64), (40, 1024, 128),
+                                   (3, 250, 16)])
+@pytest.mark.parametrize("kind,a", [("zero", 1.3), ("zero", 1.5), ("zero", -3.0), ("zero", 300.0), ("tiny", 1.5),
+                                    ("tiny", 300.0), ("inf", 0.5), ("inf", 0.01)])
+def test_pscan_coefficient_range(dev, kind, a, shape, dtype):
+    print(f"case pscan range kind={kind} a={a} shape={shape} dtype={dtype}", flush=True)
+    if kind == "tiny" and dtype == torch.float16:
+        pytest.skip("1e-30 is not an fp16 value")
+    A, X, dH = _range_inputs(kind, a, shape, dtype)
+    Ad, Xd = A.to(dev).requires_grad_(True), X.to(dev).requires_grad_(True)
+    H = parallel_scan_fn(Ad, Xd)
+    H.backward(dH.to(dev))
+    torch.cuda.synchronize()
+    ref = orc.pscan_fwd(A, X)
+    rdA, rdX = orc.pscan_bwd(A, H.detach().cpu(), dH)  # dA = G * H: from the H that the backward is given
+    if kind == "zero":
+        assert np.isfinite(ref).all() and np.isfinite(rdX).all()
+    np.testing.assert_allclose(_np(H), ref, **TOL[dtype])
+    np.testing.assert_allclose(_np(Xd.grad), rdX, **TOL[dtype])
+    np.testing.assert_allclose(_np(Ad.grad), rdA, **TOL[dtype])
+
+
 def test_pscan_matches_reference_loop_and_ignores_A0(dev):
     """parallel_scan_ref semantics (pscan.py:153-171): H_0 = X_0 whatever A_0 is."""
     g = torch.Generator().manual_seed(2)
