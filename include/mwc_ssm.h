@@ -170,7 +170,8 @@ int mwc_ssm_step(int dtype, const void* u, const void* delta, const void* A, con
                  const void* D_ssm, const void* h, const void* delta_bias, int delta_softplus, const void* z,
                  void* out, void* out_z, void* h_new, int64_t batch, int64_t dim, int64_t dstate, void* stream);
 
-/* Workspace bytes needed by mwc_pscan_fwd / mwc_pscan_bwd for these sizes. */
+/* Workspace bytes needed by mwc_pscan_fwd / mwc_pscan_bwd for these sizes; 0 for sizes they reject
+ * (negative, 2^30 or more in one dimension, more than 2^45 elements), with the reason in mwc_last_error(). */
 size_t mwc_pscan_workspace_size(int64_t nseq, int64_t seqlen, int64_t ncols);
 
 /*
@@ -192,7 +193,8 @@ int mwc_pscan_bwd(int dtype, const void* A, const void* H, const void* dH, void*
 
 /*
  * 1 if a scan of these sizes waits between tiles (bounded waits whose outcome the status functions below report),
- * 0 if it has no wait that could give up, so its status is always MWC_OK. No reference counterpart.
+ * 0 if it has no wait that could give up, so its status is always MWC_OK, and for sizes that a scan rejects. No
+ * reference counterpart.
  */
 int mwc_pscan_waits(int64_t nseq, int64_t seqlen, int64_t ncols);
 

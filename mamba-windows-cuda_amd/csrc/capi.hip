@@ -653,11 +653,30 @@ int mwc_ssm_step(int dtype, const void* u, const void* delta, const void* A, con
     return MWC_OK;
 }
 
+static int check_pscan(int dtype, int64_t nseq, int64_t seqlen, int64_t ncols) {
+    if (dtype != MWC_DTYPE_F32 && dtype != MWC_DTYPE_F16 && dtype != MWC_DTYPE_BF16)
+        return fail(MWC_ERR_INVALID_ARGUMENT, "dtype must be MWC_DTYPE_F32, MWC_DTYPE_F16 or MWC_DTYPE_BF16 (got %d)",
+                    dtype);
+    if (nseq < 0 || seqlen < 0 || ncols < 0)
+        return fail(MWC_ERR_INVALID_ARGUMENT, "negative size (nseq=%lld, seqlen=%lld, ncols=%lld)", (long long)nseq,
+                    (long long)seqlen, (long long)ncols);
+    // at most INT32_MAX tiles of at most 2^14 elements: more was never launched, and the tiling is counted in int64
+    int64_t n = 0;
+    if (nseq > INT32_MAX / 2 || seqlen > INT32_MAX / 2 || ncols > INT32_MAX / 2 ||
+        __builtin_mul_overflow(nseq * seqlen, ncols, &n) || n > int64_t(1) << 45)
+        return fail(MWC_ERR_UNSUPPORTED, "sizes beyond the supported range (nseq=%lld, seqlen=%lld, ncols=%lld)",
+                    (long long)nseq, (long long)seqlen, (long long)ncols);
+    return MWC_OK;
+}
+
+// As for the fused scan: sizes the entry points would reject need no workspace, and wait for nothing.
 size_t mwc_pscan_workspace_size(int64_t nseq, int64_t seqlen, int64_t ncols) {
+    if (check_pscan(MWC_DTYPE_F32, nseq, seqlen, ncols) != MWC_OK) return 0;
     return mwc::pscan_workspace_bytes(nseq, seqlen, ncols);
 }
 
 int mwc_pscan_waits(int64_t nseq, int64_t seqlen, int64_t ncols) {
+    if (check_pscan(MWC_DTYPE_F32, nseq, seqlen, ncols) != MWC_OK) return 0;
     return mwc::pscan_waits(nseq, seqlen, ncols) ? 1 : 0;
 }
 
@@ -668,18 +687,6 @@ static unsigned pscan_spin_limit() {
     if (!e || !*e) return mwc::kPscanSpinLimit;
     const long long v = atoll(e);
     return v < 0 ? mwc::kPscanSpinLimit : (unsigned)(v > (long long)mwc::kPscanSpinLimit ? mwc::kPscanSpinLimit : v);
-}
-
-static int check_pscan(int dtype, int64_t nseq, int64_t seqlen, int64_t ncols) {
-    if (dtype != MWC_DTYPE_F32 && dtype != MWC_DTYPE_F16 && dtype != MWC_DTYPE_BF16)
-        return fail(MWC_ERR_INVALID_ARGUMENT, "dtype must be MWC_DTYPE_F32, MWC_DTYPE_F16 or MWC_DTYPE_BF16 (got %d)",
-                    dtype);
-    if (nseq < 0 || seqlen < 0 || ncols < 0)
-        return fail(MWC_ERR_INVALID_ARGUMENT, "negative size (nseq=%lld, seqlen=%lld, ncols=%lld)", (long long)nseq,
-                    (long long)seqlen, (long long)ncols);
-    if (nseq > INT32_MAX / 2 || seqlen > INT32_MAX / 2 || ncols > INT32_MAX / 2)
-        return fail(MWC_ERR_UNSUPPORTED, "sizes beyond the supported range");
-    return MWC_OK;
 }
 
 int mwc_pscan_fwd(int dtype, const void* A, const void* X, void* H, int64_t nseq, int64_t seqlen, int64_t ncols,
@@ -714,6 +721,7 @@ int mwc_pscan_status(const void* workspace, size_t workspace_bytes, int64_t nseq
                      void* stream) {
     g_err[0] = 0;
     if (nseq <= 0 || seqlen <= 0 || ncols <= 0) return MWC_OK;  // nothing was scanned
+    if (int st = check_pscan(MWC_DTYPE_F32, nseq, seqlen, ncols)) return st;
     const size_t need = mwc::pscan_workspace_bytes(nseq, seqlen, ncols);
     if (workspace == nullptr || workspace_bytes < need)
         return fail(MWC_ERR_WORKSPACE, "scan workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
@@ -735,6 +743,7 @@ int mwc_pscan_status_async(const void* workspace, size_t workspace_bytes, int64_
         *host_word = 0;
         return MWC_OK;
     }
+    if (int st = check_pscan(MWC_DTYPE_F32, nseq, seqlen, ncols)) return st;
     const size_t need = mwc::pscan_workspace_bytes(nseq, seqlen, ncols);
     if (workspace == nullptr || workspace_bytes < need)
         return fail(MWC_ERR_WORKSPACE, "scan workspace too small: need %zu bytes, got %zu", need, workspace_bytes);

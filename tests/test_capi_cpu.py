@@ -152,6 +152,43 @@ def test_workspace_sizes_of_rejected_shapes():
             assert L.mwc_last_error(), (B, Lq, D, n)
 
 
+def test_pscan_queries_of_rejected_shapes():
+    """Sizes the parallel scan rejects need no workspace and wait for nothing: the queries return 0 and name the
+    reason (the chain count of (2^62, 1, 256) wrapped to 0, and the tiling divided by it), the status functions
+    the same refusal as the scan."""
+    from mamba_windows_cuda import _lib
+
+    L = _lib.lib()
+    word = ctypes.c_uint32(7)
+    for s in ((1 << 62, 1, 256), (1 << 61, 128, 64), (-1, 5, 5), (5, -1, 5), (5, 5, -1), (1 << 30, 1, 1),
+              (1, 1 << 30, 1), (1, 1, 1 << 30), (1 << 20, 1 << 20, 1 << 20), (1 << 29, 1 << 29, 1 << 29),
+              (1 << 15, 1 << 15, (1 << 15) + 1)):
+        assert L.mwc_pscan_workspace_size(*s) == 0, s
+        assert L.mwc_last_error(), s
+        assert L.mwc_pscan_waits(*s) == 0, s
+        refused = L.mwc_pscan_fwd(0, None, None, None, *s, None, 0, None)
+        assert refused == (1 if min(s) < 0 else 2), s
+        if min(s) > 0:
+            assert L.mwc_pscan_status(None, 0, *s, None) == refused, s
+            assert L.mwc_pscan_status_async(None, 0, *s, ctypes.byref(word), None) == refused and word.value == 7, s
+
+
+def test_pscan_waits_with_more_than_one_tile():
+    """A scan waits from the step on at which it has a second tile along L: 257 steps at 16 columns or fewer, 129
+    beyond. Empty scans wait for nothing and need nothing."""
+    from mamba_windows_cuda import _lib
+
+    L = _lib.lib()
+    for ncols, steps in ((1, 256), (8, 256), (9, 256), (16, 256), (17, 128), (32, 128), (33, 128), (64, 128),
+                         (66, 128), (1024, 128)):
+        for nseq in (1, 3, 5000):
+            assert L.mwc_pscan_waits(nseq, 1, ncols) == 0
+            assert L.mwc_pscan_waits(nseq, steps, ncols) == 0
+            assert L.mwc_pscan_waits(nseq, steps + 1, ncols) == 1
+    for s in ((0, 5, 5), (5, 0, 5), (5, 5, 0)):
+        assert L.mwc_pscan_waits(*s) == 0 and L.mwc_pscan_workspace_size(*s) == 0
+
+
 def test_status_strings_and_ckpt_count():
     from mamba_windows_cuda import _lib
 
