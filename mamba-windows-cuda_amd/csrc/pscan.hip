@@ -64,13 +64,14 @@ PscanGeom geom(int64_t nseq, int64_t seqlen, int64_t ncols, int vec) {
     g.cw = lanes <= 8 ? 8 : lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
     g.ncolblk = (int)((lanes + g.cw - 1) / g.cw);
     g.nltile = (int)((seqlen + tile_steps(g.cw) - 1) / tile_steps(g.cw));
-    const int64_t nchains = nseq * g.ncolblk, most = ticket_chains(g.cw, nchains * g.nltile);
+    const bool one = g.nltile == 1;  // no tickets and no flags: the error word is all that such a scan uses
+    const int64_t nchains = nseq * g.ncolblk, most = one ? 1 : ticket_chains(g.cw, nchains * g.nltile);
     g.ngroups = (nchains + most - 1) / most;
     g.gchains = (int)((nchains + g.ngroups - 1) / g.ngroups);
     g.ngroups = (nchains + g.gchains - 1) / g.gchains;
     g.nblocks = g.ngroups * g.gchains * g.nltile;
-    g.flags_offset = (size_t)(1 + g.ngroups) * kTicketStride * sizeof(unsigned);
-    g.bytes = g.flags_offset + (size_t)nseq * g.ncolblk * g.nltile * g.cw * vec * 2 * sizeof(uint64_t);
+    g.flags_offset = (size_t)(1 + (one ? 0 : g.ngroups)) * kTicketStride * sizeof(unsigned);
+    g.bytes = g.flags_offset + (one ? 0 : (size_t)nchains * g.nltile * g.cw * vec * 2 * sizeof(uint64_t));
     return g;
 }
 
@@ -168,8 +169,8 @@ __global__ void __launch_bounds__(kThreads, CW == 64 ? 3 : CW == 8 ? 8 : REV ? 5
     const int64_t chain0 = (int64_t)group * gchains;
     const int gw = (int)min((int64_t)gchains, nchains - chain0);
     const int nltile = (L + TS - 1) / TS;
-    if (threadIdx.x == 0) {  // one tile along L: nothing waits, so any order does
-        s_tile = nltile > 1 ? (int)atomicAdd(tickets + (size_t)group * kTicketStride, 1u) : (int)(blockIdx.x / ngroups);
+    if (threadIdx.x == 0) {  // one tile along L: nothing waits, a group is one tile
+        s_tile = nltile > 1 ? (int)atomicAdd(tickets + (size_t)group * kTicketStride, 1u) : 0;
         s_wide = 0;
     }
     if (nltile == 1 && blockIdx.x == 0 && threadIdx.x == 0) *err = 0;  // nor is the workspace cleared

@@ -189,6 +189,17 @@ def test_pscan_waits_with_more_than_one_tile():
         assert L.mwc_pscan_waits(*s) == 0 and L.mwc_pscan_workspace_size(*s) == 0
 
 
+def test_pscan_workspace_of_one_tile():
+    """One tile along L uses the error word alone; the second one brings tickets and flags, 16 bytes a column."""
+    from mamba_windows_cuda import _lib
+
+    L = _lib.lib()
+    for s in ((1, 1, 1), (1000000, 4, 8), (500, 256, 16), (70, 128, 1024), (3, 128, 1050)):
+        assert L.mwc_pscan_workspace_size(*s) == 64, s
+    for nseq, steps, ncols in ((500, 257, 16), (70, 129, 1024), (3, 129, 1050)):
+        assert L.mwc_pscan_workspace_size(nseq, steps, ncols) > 2 * 16 * nseq * ncols
+
+
 def test_status_strings_and_ckpt_count():
     from mamba_windows_cuda import _lib
 

@@ -65,12 +65,12 @@ def test_pscan_narrow_sequences(dev, shape, dtype):
 
 
 # Pairs of 16-bit columns: 33 to 64 and more, whole and ragged column blocks, and the odd widths, fewer tiles and
-# misaligned tensors that stay with single columns. The 68 column blocks
-# of 17 tiles share tickets in groups of 34, the 65 in groups of 33 and 32.
+# misaligned tensors that stay with single columns. (1101, 33, .) have one tile along L and more than 1024 in all.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shape,offset", [((128, 5, 34), 0), ((130, 128, 64), 0), ((64, 130, 66), 0), ((64, 257, 62), 1),
                                           ((3, 2049, 382), 0), ((3, 2049, 382), 1), ((3, 2049, 381), 0),
-                                          ((2, 300, 1050), 0), ((4, 2100, 1050), 0), ((65, 2100, 64), 1), ((1, 129, 130), 0)])
+                                          ((2, 300, 1050), 0), ((4, 2100, 1050), 0), ((65, 2100, 64), 1), ((1, 129, 130), 0),
+                                          ((1101, 33, 64), 0), ((1101, 33, 128), 0)])
 def test_pscan_column_pairs(dev, shape, offset, dtype):
     print(f"case pscan pairs shape={shape} offset={offset} dtype={dtype}", flush=True)
     g = torch.Generator().manual_seed(shape[0] + shape[1])
