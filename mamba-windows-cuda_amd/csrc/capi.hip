@@ -387,22 +387,25 @@ SegPlan plan_rules(const SsmShape& s, bool bwd) {
     return h.nseg > 0 && (x_forced > 0 || th < t * 0.98) ? h : p;
 }
 
-// The plan of the last shape that this thread asked for is kept, per direction: a call asks for it three times, and a
-// loop for the same shape each time. Overrides (tuning and tests) are read on every call.
+// The plans of the shapes that this thread asked for last are kept, per direction (64 of them, one per slot): a call
+// asks for its plan three times, and a program for the same few shapes over and over. Overrides (tuning and tests) are
+// read on every call.
 SegPlan plan_dir(const SsmShape& s, bool bwd) {
     for (const char* e : {"MWC_SPL", "MWC_NSEG", "MWC_CFOLD", "MWC_NSPLIT"})
         if (getenv(e) != nullptr) return plan_rules(s, bwd);
-    static thread_local struct {
-        SsmShape s{-1, -1, -1, 0};
-        SegPlan p;
-    } last[2];
-    auto& l = last[bwd];
-    if (l.s.batch != s.batch || l.s.seqlen != s.seqlen || l.s.dim != s.dim || l.s.nstate != s.nstate) {
+    struct Kept {
+        SsmShape s{-1, -1, -1, 0};  // no shape
+        SegPlan p{};
+    };
+    static thread_local Kept kept[2][64];
+    const uint64_t h = ((uint64_t)s.batch * 31 + (uint64_t)s.seqlen) * 1000003 + (uint64_t)s.dim * 127 + s.nstate;
+    Kept& k = kept[bwd][(h * 0x9e3779b97f4a7c15ull) >> 58];
+    if (k.s.nstate != s.nstate || k.s.batch != s.batch || k.s.seqlen != s.seqlen || k.s.dim != s.dim) {
         const SegPlan p = plan_rules(s, bwd);
-        l.p = p.nfull > 0 ? p : small_grid_plan(s, bwd, p);
-        l.s = s;
+        k.p = p.nfull > 0 ? p : small_grid_plan(s, bwd, p);
+        k.s = s;
     }
-    return l.p;
+    return k.p;
 }
 
 }  // namespace

@@ -200,6 +200,56 @@ def test_pscan_workspace_of_one_tile():
         assert L.mwc_pscan_workspace_size(nseq, steps, ncols) > 2 * 16 * nseq * ncols
 
 
+PLAN_SHAPES = [(B, Lq, D, n) for B in (1, 3, 8) for Lq in (17, 64, 333, 1024, 4000) for D in (64, 100, 777, 2560)
+               for n in (8, 16, 32, 64)]
+
+
+def _plan_sizes(L, shapes):
+    return [(L.mwc_ssm_fwd_workspace_size(*s), L.mwc_ssm_bwd_workspace_size(*s)) for s in shapes]
+
+
+def test_kept_plans_are_those_of_their_shapes():
+    """The planner keeps the plans of recent shapes per thread: more shapes than it keeps, in any order and in a
+    thread that has kept none, give the same workspace sizes."""
+    import random
+    import threading
+
+    from mamba_windows_cuda import _lib
+
+    L = _lib.lib()
+    want = dict(zip(PLAN_SHAPES, _plan_sizes(L, PLAN_SHAPES)))
+    for seed in range(3):
+        order = random.Random(seed).choices(PLAN_SHAPES, k=500)
+        assert _plan_sizes(L, order) == [want[s] for s in order]
+        got = []
+        t = threading.Thread(target=lambda: got.extend(_plan_sizes(L, order)))
+        t.start()
+        t.join()
+        assert got == [want[s] for s in order]
+
+
+def test_alternating_shapes_do_not_plan_again():
+    """Two shapes in turn cost a query what one shape does (with one plan kept per thread it took five times as
+    long, on every change of a prompt's length). Best of several runs, within a factor of two."""
+    import time
+
+    from mamba_windows_cuda import _lib
+
+    L = _lib.lib()
+
+    def best(shapes, calls=2000):
+        t = []
+        for _ in range(15):
+            t0 = time.perf_counter()
+            for i in range(calls):
+                L.mwc_ssm_fwd_workspace_size(*shapes[i % 2])
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    a, b = (1, 1024, 256, 16), (1, 1040, 256, 16)
+    assert best((a, b)) < 2.0 * best((a, a))
+
+
 def test_status_strings_and_ckpt_count():
     from mamba_windows_cuda import _lib
 
