@@ -253,103 +253,154 @@ SegPlan fill_plan(const SsmShape& s, bool bwd, int spl, int cap_main, int cap_ca
     return SegPlan{spl, 0, 0, 0, 0};
 }
 
-// Small grids: modelled times in us. A pass costs its chunks at the rate of the waves that share a SIMD plus a
-// prologue for each round of workgroups, a carry pass its launch besides, and a main workgroup `fold` for each carry
-// that it folds into its start, one dependent load after the other; chunk times are those of a lone wave. Fitted to
-// every (states per lane, segments, carry split) measured at 31 shapes from (1, 256, 64) to (8, 2048, 1536) with N = 8,
-// 16, 32 and 64, in both directions. Its choice, where it is modelled at under 0.9 (backward 0.95) of the other rules'
-// plan, is 4.9% (forward) and 2.1% (backward) above the fastest plan of a shape on average against 13.5% and 8.8%
-// without it; at 0.95 some forwards got 2-4% slower. At 9 shapes it was not fitted to it gained 10% on average,
-// (6, 400, 300) N=32 backward 51 -> 36 us at best and (5, 100, 2000) 30.7 -> 32.3 at worst. The rules cut few channels too finely: they price
-// no fold, so (1, 1024, 256) fp32 ran 16 segments with carries split 4 ways, 19.9 and 28.4 us against 13.3 and 20.2.
+// Small grids: modelled times in us. A pass costs its chunks at the rate of the waves that share a SIMD (chunk times
+// are those of a lone wave) plus a prologue for each round of workgroups, which grows with their number on a CU; a
+// carry pass its launch besides, and a main workgroup `fold` for each carry that it folds into its start, one dependent
+// load after the other. The backward's finishing kernel sums the dB/dC partials of the channel groups and the dA/dD
+// partials of the segments, one after the other, and reads them all. Fitted by profiles/plan_model.py to 10,855 plans
+// in each direction at 284 shapes (profiles/plan_sweep.jsonl). The model's choice, taken where it is modelled at under
+// 0.97 of the other rules' plan, is 1.1% (forward) and 1.4% (backward) above the fastest plan of a shape on average
+// against 15.6% and 8.4% of the rules; without a margin 1.0% and 0.9%, but up to 7% slower than the rules at single
+// shapes. At 300 other shapes calls take 0.85 and 0.91 times what the rules' plans take, no shape of them over 1.04 but
+// by noise. Without the finishing kernel and the growing prologues the fit put their cost into the rates (four waves
+// faster than one) and picked plans up to 28% slower than the rules': (1, 64, 2560) backward 19.5 -> 25.0 us, now 19.3.
 struct CostModel {
     double fold, launch;
+    double fin_group, fin_rows, fin_mb;  // finishing kernel: per channel group, per 32 rows of partials, per MB
     struct {
-        double main, carry;        // prologues
+        double main, main_more;    // prologue of a lone workgroup on its CU, and what each further one adds
+        double carry, carry_more;  // the carry pass's
         double rate[4], crate[4];  // relative rate of 2, 3, 4 and 6 or more waves per SIMD
     } spl[3];                      // 1, 2 and 4 states per lane
     struct {
         double main, carry;  // one chunk of a lone wave
     } chunk[4][3];           // by state count and states per lane; 0: not measured
 };
-const CostModel kFwdCost = {
-    0.135, 1.76,
-    {{3.80, 2.27, {1.44, 1.87, 2.14, 2.73}, {1.49, 1.66, 1.75, 2.02}},
-     {4.07, 2.65, {1.62, 2.17, 2.37, 2.47}, {1.02, 1.12, 1.19, 1.27}},
-     {9.47, 3.96, {1.49, 1.71, 1.91, 2.01}, {1.29, 1.32, 1.61, 1.71}}},
-    {{{0.69, 0.30}, {0.87, 0.54}, {0, 0}},
-     {{0.62, 0.37}, {0.86, 0.46}, {0, 0}},
-     {{0, 0}, {0.90, 0.44}, {1.32, 0.59}},
-     {{0, 0}, {0, 0}, {1.51, 0.53}}}};
-const CostModel kBwdCost = {
-    0.133, 3.77,
-    {{6.44, 1.88, {1.43, 1.78, 2.00, 2.10}, {1.38, 1.61, 1.77, 3.28}},
-     {5.69, 3.27, {1.47, 1.84, 2.04, 2.14}, {1.03, 1.20, 1.36, 1.50}},
-     {8.03, 6.51, {1.42, 1.72, 1.92, 2.02}, {1.68, 2.24, 4.26, 4.36}}},
-    {{{1.52, 0.28}, {2.13, 0.53}, {0, 0}},
-     {{1.50, 0.26}, {2.01, 0.46}, {0, 0}},
-     {{0, 0}, {2.04, 0.53}, {3.20, 0.93}},
-     {{0, 0}, {0, 0}, {4.13, 0.43}}}};
+constexpr CostModel kFwdCost = {
+    0.141, 2.11,
+    0.000, 0.00, 0.00,
+    {{3.10, 0.42, 0.32, 0.46, {1.73, 2.19, 2.54, 2.87}, {2.00, 2.73, 3.11, 4.22}},
+     {3.14, 0.72, 0.46, 0.84, {1.72, 2.21, 1.88, 2.51}, {1.73, 2.26, 2.55, 3.13}},
+     {3.13, 1.33, 0.81, 1.37, {1.73, 2.32, 2.24, 2.41}, {1.54, 1.80, 2.09, 2.90}}},
+    {{{0.81, 0.59}, {1.04, 0.86}, {0, 0}},
+     {{0.73, 0.58}, {0.92, 0.79}, {0, 0}},
+     {{0, 0}, {0.92, 0.75}, {1.44, 1.15}},
+     {{0, 0}, {0, 0}, {1.61, 1.16}}}};
+constexpr CostModel kBwdCost = {
+    0.199, 2.51,
+    0.084, 1.14, 0.21,
+    {{4.44, 0.39, 0.30, 0.26, {1.82, 2.38, 2.75, 2.96}, {1.75, 2.43, 3.06, 4.53}},
+     {4.41, 0.61, 0.62, 0.66, {1.77, 2.29, 2.08, 1.77}, {1.51, 2.17, 2.84, 2.90}},
+     {2.61, 2.00, 3.48, 0.31, {1.71, 1.84, 2.40, 3.27}, {1.43, 1.84, 2.09, 3.13}}},
+    {{{1.76, 0.58}, {2.52, 0.77}, {0, 0}},
+     {{1.60, 0.51}, {2.23, 0.68}, {0, 0}},
+     {{0, 0}, {2.14, 0.87}, {3.46, 1.00}},
+     {{0, 0}, {0, 0}, {3.75, 0.99}}}};
+constexpr double kModelMargin = 0.97;  // see above
 
-double wave_rate(const double* r, int64_t q) {
+constexpr double wave_rate(const double* r, int q) {
     return q <= 1 ? 1.0 : q >= 6 ? r[3] : q == 5 ? 0.5 * (r[2] + r[3]) : r[q - 2];
 }
+// More waves on a SIMD never finish sooner, and q of them do at most q times the work of one: without this a fit
+// takes a cost that it has no term for out of the rates, and then favours grids that only look cheaper.
+constexpr bool rates_possible(const double* r) {
+    for (int q = 1; q < 8; ++q)
+        if ((q + 1) / wave_rate(r, q + 1) < q / wave_rate(r, q) || wave_rate(r, q + 1) > q + 1) return false;
+    return true;
+}
+constexpr bool rates_possible(const CostModel& m) {
+    for (int i = 0; i < 3; ++i)
+        if (!rates_possible(m.spl[i].rate) || !rates_possible(m.spl[i].crate)) return false;
+    return true;
+}
+static_assert(rates_possible(kFwdCost) && rates_possible(kBwdCost), "the time of a pass grows with its workgroups");
 
 // pass_time with the model's costs
-double pass_us(int64_t wgs, int64_t chunks, int cap, double chunk, double prologue, const double* rate) {
+double pass_us(int wgs, int chunks, int cap, double chunk, double prologue, double more, const double* rate) {
     if (wgs <= 0 || chunks <= 0) return 0.0;
-    const int64_t full = wgs / ((int64_t)kCUs * cap), rem = wgs - full * kCUs * cap;
-    double t = (double)full * ((double)chunks * chunk * cap / wave_rate(rate, cap) + prologue);
-    if (rem > 0) {
-        const int64_t q = (rem + kCUs - 1) / kCUs;
-        t += (double)chunks * chunk * q / wave_rate(rate, q) + prologue;
-    }
+    const int per_cu = (wgs + kCUs - 1) / kCUs, full = wgs / kCUs / cap, q = per_cu - full * cap;
+    double t = 0.0;
+    if (full > 0) t = full * (chunks * chunk * cap / wave_rate(rate, cap) + prologue + more * (cap - 1));
+    if (q > 0) t += chunks * chunk * q / wave_rate(rate, q) + prologue + more * (q - 1);
     return t;
 }
 
-double plan_us(const SsmShape& s, bool bwd, const SegPlan& p, int cap_main, int cap_carry) {
-    const CostModel& m = bwd ? kBwdCost : kFwdCost;
-    const int ni = s.nstate == 8 ? 0 : s.nstate == 16 ? 1 : s.nstate == 32 ? 2 : 3, si = p.spl == 4 ? 2 : p.spl - 1;
-    const auto& c = m.chunk[ni][si];
-    const int64_t w1 = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl));
-    double t = pass_us(w1 * p.nseg, p.cps, cap_main, c.main, m.spl[si].main, m.spl[si].rate);
-    if (p.nseg > 1)
-        t += m.launch + pass_us(w1 * p.ncar, p.cps / p.cfold, cap_carry, c.carry, m.spl[si].carry, m.spl[si].crate) +
-             m.fold * (bwd ? p.ncar : (p.nseg - 1) * p.cfold);
-    return t;
-}
+int state_index(int ns) { return ns == 8 ? 0 : ns == 16 ? 1 : ns == 32 ? 2 : 3; }
+int lane_index(int spl) { return spl == 4 ? 2 : spl - 1; }
+
+// Modelled plans of one shape and direction at one count of states per lane
+struct PlanCost {
+    const SsmShape& s;
+    const CostModel& m;
+    const bool bwd;
+    const int si, wgs, cap_main, cap_carry;  // wgs: workgroups of one segment
+    const double main_chunk, carry_chunk, fin, fin_rows;
+    PlanCost(const SsmShape& s_, bool bwd_, int spl)
+        : s(s_), m(bwd_ ? kBwdCost : kFwdCost), bwd(bwd_), si(lane_index(spl)),
+          wgs((int)(s.batch * ((s.dim + cpb_of(s.nstate, spl) - 1) / cpb_of(s.nstate, spl)))),
+          cap_main(bwd ? bwd_cap(s.nstate, spl) : fwd_cap(s.nstate, spl)),
+          cap_carry(bwd ? bwd_carry_cap(s.nstate, spl) : fwd_carry_cap(s.nstate, spl)),
+          main_chunk(m.chunk[state_index(s.nstate)][si].main), carry_chunk(m.chunk[state_index(s.nstate)][si].carry),
+          fin(m.fin_group * (wgs / (double)s.batch)), fin_rows(m.fin_rows) {}
+    // the main pass and the finishing kernel of nseg segments of cps chunks
+    double main_us(int nseg, int cps) const {
+        const double read = m.fin_mb * 8e-6 * wgs * (double)s.seqlen * s.nstate;
+        return pass_us(wgs * nseg, cps, cap_main, main_chunk, m.spl[si].main, m.spl[si].main_more,
+                       m.spl[si].rate) + read +
+               std::max(fin, fin_rows * (double)((nseg * s.batch + 31) / 32));
+    }
+    // a lower bound of the plans at about n segments of at least `per` chunks
+    double least_us(int n, int per) const {
+        return fin + m.spl[si].main + per * main_chunk +
+               (n > 1 ? m.launch + m.spl[si].carry + (per * carry_chunk + (n - 2) * m.fold) * 0.25 : 0.0);
+    }
+    // what the carries of ncar carry segments of ccps chunks add to that, of which a workgroup folds `folds`
+    double carry_us(int ncar, int ccps, int folds) const {
+        return m.launch + m.fold * folds +
+               pass_us(wgs * ncar, ccps, cap_carry, carry_chunk, m.spl[si].carry, m.spl[si].carry_more,
+                       m.spl[si].crate);
+    }
+};
 
 // The model's plan where it undercuts `p` clearly, else `p`. Never one whose carries need more scratch than `p`'s and
-// than the scratch of mwc_ssm_fwd_noalloc, so that no size which that entry point takes gets refused.
+// than the scratch of mwc_ssm_fwd_noalloc, so that no size which that entry point takes gets refused. (The backward's
+// partials may grow with its segments: its workspace is 1.6 times that of `p` at most, and smaller at most shapes.)
 SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
-    const int64_t nck = (s.seqlen + kCkptSteps - 1) / kCkptSteps;
+    const int64_t chunks = (s.seqlen + kCkptSteps - 1) / kCkptSteps;
     const int64_t w1 = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl));
-    const int ni = s.nstate == 8 ? 0 : s.nstate == 16 ? 1 : s.nstate == 32 ? 2 : 3;
-    if (w1 <= 0 || nck < 2 || w1 >= (int64_t)kCUs * 3 / 2 || kFwdCost.chunk[ni][p.spl == 4 ? 2 : p.spl - 1].main == 0)
-        return p;
-    auto caps = [&](int spl, int& cm, int& cc) {
-        cm = bwd ? bwd_cap(s.nstate, spl) : fwd_cap(s.nstate, spl);
-        cc = bwd ? bwd_carry_cap(s.nstate, spl) : fwd_carry_cap(s.nstate, spl);
-    };
-    int cm = 0, cc = 0;
-    caps(p.spl, cm, cc);
+    const auto& known = kFwdCost.chunk[state_index(s.nstate)];
+    // up to 1.5 workgroups a CU, which is where the measurements end
+    if (w1 <= 0 || chunks < 2 || w1 >= (int64_t)kCUs * 3 / 2 || known[lane_index(p.spl)].main == 0) return p;
+    const int nck = (int)chunks;
     SegPlan best = p;
-    double best_t = (bwd ? 0.95 : 0.9) * plan_us(s, bwd, p, cm, cc);
+    const PlanCost own(s, bwd, p.spl);
+    double best_t = own.main_us(p.nseg, p.cps);
+    if (p.nseg > 1)
+        best_t += own.carry_us(p.ncar, p.cps / p.cfold, bwd ? p.ncar : (p.nseg - 1) * p.cfold);
+    best_t *= kModelMargin;
     const size_t most = std::max<size_t>(carry_bytes(s, p), MWC_NOALLOC_SCRATCH_BYTES / 2);
     for (int spl = 1; spl <= 4; spl *= 2) {
-        if (kFwdCost.chunk[ni][spl == 4 ? 2 : spl - 1].main == 0) continue;
-        caps(spl, cm, cc);
-        const int64_t ws = s.batch * ((s.dim + cpb_of(s.nstate, spl) - 1) / cpb_of(s.nstate, spl));
+        if (known[lane_index(spl)].main == 0) continue;
+        const PlanCost c(s, bwd, spl);
         for (int n : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48}) {
+            const int per = (nck + n - 1) / n;
+            if (n > 1 && per < 2) break;  // segments of one chunk run longer than modelled
+            if (c.least_us(n, per) >= best_t) continue;
+            int cps = 0, nseg = 0;
+            double main = 0.0;
             for (int f = 1; f <= (n > 1 ? 4 : 1); f *= 2) {
-                const int64_t cps = ((nck + n - 1) / n + f - 1) / f * f, nseg = (nck + cps - 1) / cps, ccps = cps / f;
-                if (n > 1 && (nseg < 2 || cps < 2)) continue;  // segments of one chunk run longer than modelled
-                const int64_t ncar = nseg < 2 ? 0 : bwd ? (nck - cps + ccps - 1) / ccps : (nseg - 1) * f;
-                const SegPlan q{spl, (int)nseg, (int)cps, f, (int)ncar};
-                if (ws * nseg > INT32_MAX / 2 || carry_bytes(s, q) > most) continue;
-                double t = plan_us(s, bwd, q, cm, cc);
-                if (bwd && nseg < 2) t *= 0.95 / 0.9;  // so do unsplit backwards
-                if (t < best_t) {
+                const int up = (per + f - 1) & -f, ccps = up / f;  // f: 1, 2 or 4
+                if (up != cps) {
+                    cps = up;
+                    nseg = (nck + cps - 1) / cps;
+                    main = c.main_us(nseg, cps);
+                }
+                if (n > 1 && nseg < 2) break;
+                if (main >= best_t) continue;
+                const int ncar = nseg < 2 ? 0 : bwd ? (nck - cps + ccps - 1) / ccps : (nseg - 1) * f;
+                const SegPlan q{spl, nseg, cps, f, ncar};
+                const double t = nseg < 2 ? main : main + c.carry_us(ncar, ccps, bwd ? ncar : (nseg - 1) * f);
+                if (t < best_t && carry_bytes(s, q) <= most) {
                     best_t = t;
                     best = q;
                 }

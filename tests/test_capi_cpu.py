@@ -250,6 +250,34 @@ def test_alternating_shapes_do_not_plan_again():
     assert best((a, b)) < 2.0 * best((a, a))
 
 
+def test_planner_small_grids_against_the_rules(monkeypatch):
+    """Small grids take the plan of a cost model where it undercuts the planner's rules (which a state-per-lane override
+    that names no supported count leaves alone). The forward's scratch never exceeds both the rules' and what
+    mwc_ssm_fwd_noalloc has, the backward's grows within bounds, and short backwards do not run unsplit at the fewest
+    states per lane, with twice the dB/dC partials to sum: measured 14 to 28% slower than the rules' plans, but taken by
+    a model without the finishing kernel."""
+    from mamba_windows_cuda import _lib
+    from tests.test_gpu_random import SMALL_CASES
+
+    L = _lib.lib()
+    short = {(1, 64, 2560, 16): 1, (2, 80, 1356, 16): 1, (3, 109, 2910, 16): 1, (3, 64, 128, 32): 2}
+    small = [(c["B"], c["L"], c["D"], c["n"]) for c in SMALL_CASES]
+    shapes = PLAN_SHAPES + list(short) + small
+    model = dict(zip(shapes, _plan_sizes(L, shapes)))
+    monkeypatch.setenv("MWC_SPL", "0")
+    rules = dict(zip(shapes, _plan_sizes(L, shapes)))
+    scratch = 32 << 20  # MWC_NOALLOC_SCRATCH_BYTES
+    for s in shapes:
+        assert model[s][0] <= max(rules[s][0], scratch), s
+        assert model[s][1] <= 1.75 * rules[s][1], s
+    monkeypatch.setenv("MWC_NSEG", "1")
+    for s, spl in short.items():
+        monkeypatch.setenv("MWC_SPL", str(spl))
+        assert model[s][1] != L.mwc_ssm_bwd_workspace_size(*s), s
+    assert sum(model[s] != rules[s] for s in small) >= 4  # the model's plans are what test_planner_small_grids runs
+    assert sum(model[s] != rules[s] for s in PLAN_SHAPES) >= len(PLAN_SHAPES) // 4
+
+
 def test_status_strings_and_ckpt_count():
     from mamba_windows_cuda import _lib
 
