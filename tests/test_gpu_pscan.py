@@ -65,11 +65,15 @@ def test_pscan_narrow_sequences(dev, shape, dtype):
 
 
 # Pairs of 16-bit columns: 33 to 64 and more, whole and ragged column blocks, and the odd widths, fewer tiles and
-# misaligned tensors that stay with single columns. (1101, 33, .) have one tile along L and more than 1024 in all.
+# misaligned tensors that stay with single columns. Tickets are shared from 1024 tiles on: (7, 2100, 1282) in 16 bits
+# has 77 pair blocks of 17 tiles in groups of 39 and 38, in fp32 147 blocks in groups of 49; (4, 2100, 1050) shares them
+# in fp32 only (68 blocks in groups of 34), (65, 2100, 64) in every type, with single columns (33 and 32). (1101, 33, .)
+# have one tile along L and more than 1024 in all.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("shape,offset", [((128, 5, 34), 0), ((130, 128, 64), 0), ((64, 130, 66), 0), ((64, 257, 62), 1),
-                                          ((3, 2049, 382), 0), ((3, 2049, 382), 1), ((3, 2049, 381), 0),
-                                          ((2, 300, 1050), 0), ((4, 2100, 1050), 0), ((65, 2100, 64), 1), ((1, 129, 130), 0),
+@pytest.mark.parametrize("shape,offset", [((128, 5, 34), 0), ((130, 128, 64), 0), ((64, 130, 66), 0),
+                                          ((64, 257, 62), 1), ((3, 2049, 382), 0), ((3, 2049, 382), 1), ((3, 2049, 381), 0),
+                                          ((2, 300, 1050), 0), ((4, 2100, 1050), 0), ((7, 2100, 1282), 0),
+                                          ((65, 2100, 64), 1), ((1, 129, 130), 0),
                                           ((1101, 33, 64), 0), ((1101, 33, 128), 0)])
 def test_pscan_column_pairs(dev, shape, offset, dtype):
     print(f"case pscan pairs shape={shape} offset={offset} dtype={dtype}", flush=True)
@@ -128,7 +132,7 @@ def _range_inputs(kind, a, shape, dtype):
 def test_pscan_coefficient_range(dev, kind, a, shape, dtype):
     print(f"case pscan range kind={kind} a={a} shape={shape} dtype={dtype}", flush=True)
     if kind == "tiny" and dtype == torch.float16:
-        pytest.skip("1e-30 is not an fp16 value")
+        dtype = torch.float32  # 1e-30 is not an fp16 value
     A, X, dH = _range_inputs(kind, a, shape, dtype)
     Ad, Xd = A.to(dev).requires_grad_(True), X.to(dev).requires_grad_(True)
     H = parallel_scan_fn(Ad, Xd)
