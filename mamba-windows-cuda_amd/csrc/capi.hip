@@ -261,8 +261,8 @@ SegPlan fill_plan(const SsmShape& s, bool bwd, int spl, int cap_main, int cap_ca
 // in each direction at 284 shapes (profiles/plan_sweep.jsonl). The model's choice, taken where it is modelled at under
 // 0.97 of the other rules' plan, is 1.1% (forward) and 1.4% (backward) above the fastest plan of a shape on average
 // against 15.6% and 8.4% of the rules; without a margin 1.0% and 0.9%, but up to 7% slower than the rules at single
-// shapes. At 300 other shapes calls take 0.85 and 0.91 times what the rules' plans take, no shape of them over 1.04 but
-// by noise. Without the finishing kernel and the growing prologues the fit put their cost into the rates (four waves
+// shapes. At 300 other shapes calls take 0.85 and 0.91 times what the rules' plans take, none of them more than
+// 1.07. Without the finishing kernel and the growing prologues the fit put their cost into the rates (four waves
 // faster than one) and picked plans up to 28% slower than the rules': (1, 64, 2560) backward 19.5 -> 25.0 us, now 19.3.
 struct CostModel {
     double fold, launch;
@@ -364,7 +364,8 @@ struct PlanCost {
 
 // The model's plan where it undercuts `p` clearly, else `p`. Never one whose carries need more scratch than `p`'s and
 // than the scratch of mwc_ssm_fwd_noalloc, so that no size which that entry point takes gets refused. (The backward's
-// partials may grow with its segments: its workspace is 1.6 times that of `p` at most, and smaller at most shapes.)
+// partials follow its segments and states per lane: of 6,000 random shapes its workspace is at most 1.6 times that of
+// `p`, and under 0.8 times at 1,842.)
 SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
     const int64_t chunks = (s.seqlen + kCkptSteps - 1) / kCkptSteps;
     const int64_t w1 = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl));

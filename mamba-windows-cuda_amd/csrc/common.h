@@ -293,7 +293,8 @@ template <int G, int V> __device__ __forceinline__ float reduce_scatter(float (&
 // bits 4 and 5 swap rows / halves of a register pair (v_permlane16_swap_b32, v_permlane32_swap_b32),
 // bits 3 and 2 are DPP reads of lane +-8 / +-4 whose halves are selected by bank masks. So each level
 // costs two instructions per value it leaves (no selects), and a last single-value level on a DPP bit
-// costs one. Level order: the permlane bits first (while two or more values remain), then bits 3, 2.
+// costs one. Level order: the DPP bits 3 and 2 first, the cheapest exchange where there are the most pairs (see
+// hi_bit), then the permlane bits 4 and 5.
 // At a level on lane bit b the lanes with bit b = 0 keep the even values (2q) and the others the odd
 // ones (2q+1), each adding its partner's copy; the lane returns the group sum of value
 // rs_hi_index<CPW, V>(lane). The clang builtins for the permlane swaps drop their second result in this

@@ -7,8 +7,8 @@
 // dA_t = G_t*H_{t-1} for t >= 1 and dA_0 = 0.
 //
 // Design: one pass over HBM (12 B/element forward, 20 B/element backward).
-// A tile is TL consecutive steps x CW columns; each thread owns one column and
-// RUN consecutive steps held in VGPRs. Thread runs are combined inside the
+// A tile is TS consecutive steps x CW threads across; each thread owns one column
+// (a pair of them in wide 16-bit scans) and RUN consecutive steps held in VGPRs. Thread runs are combined inside the
 // tile through LDS; tiles along L are chained with a decoupled look-back:
 // each tile publishes its aggregate map h -> a*h + b per column, then its
 // inclusive prefix once known, as 64-bit (status << 32 | fp32 bits) words so
@@ -40,6 +40,8 @@ constexpr int kThreads = 256;
 // 134 us (forward, adjoint) against 80 and 139 with 128, (1, 30000, 16) 15 us against 19; 512 steps at 8 columns made
 // (20000, 200, 8) fp16 56 us instead of 40.
 constexpr int tile_steps(int cw) { return cw <= 16 ? 256 : 128; }
+// Waves a SIMD that the kernels are compiled to fit. 80 VGPRs leave 6, which narrow forwards would exceed by two.
+constexpr int scan_waves(int cw, bool rev) { return cw == 64 ? 3 : cw == 8 ? 8 : rev ? 5 : 6; }
 constexpr uint32_t kStAgg = 1, kStInc = 2;
 constexpr int kTicketStride = 16;  // words: a ticket has a cache line of its own
 // Column blocks (chains of tiles along L) that share a ticket. One ticket for all tiles serves one in about 12 ns, which
@@ -149,15 +151,13 @@ template <typename T, int V> __device__ __forceinline__ void row_st(T* p, const 
 
 // REV = false: forward scan of X with coefficients A (A_0 ignored) into Out.
 // REV = true : adjoint; X = dH, Out = dX, Hs = forward H, dAo = dA.
-// A thread owns V adjacent columns (2: 16-bit pairs). Waves: 80 VGPRs leave 6 a SIMD, which the exponents' code would
-// exceed by two registers; the adjoint's 16 more values fit 5.
+// A thread owns V adjacent columns (2: 16-bit pairs).
 template <typename T, int CW, int V, bool REV>
-__global__ void __launch_bounds__(kThreads, CW == 64 ? 3 : CW == 8 ? 8 : REV ? 5 : 6) pscan_kernel(const T* __restrict__ A, const T* __restrict__ X,
-                                                         const T* __restrict__ Hs, T* __restrict__ Out,
-                                                         T* __restrict__ dAo, uint64_t* __restrict__ flags,
-                                                         unsigned* __restrict__ tickets, unsigned* __restrict__ err,
-                                                         int L, int ncols, int ncolblk, int64_t nchains, int gchains,
-                                                         unsigned ngroups, unsigned spin_limit) {
+__global__ void __launch_bounds__(kThreads, scan_waves(CW, REV))
+pscan_kernel(const T* __restrict__ A, const T* __restrict__ X, const T* __restrict__ Hs, T* __restrict__ Out,
+             T* __restrict__ dAo, uint64_t* __restrict__ flags, unsigned* __restrict__ tickets,
+             unsigned* __restrict__ err, int L, int ncols, int ncolblk, int64_t nchains, int gchains,
+             unsigned ngroups, unsigned spin_limit) {
     constexpr int R = kThreads / CW;     // thread rows per tile
     constexpr int TS = tile_steps(CW), RUN = TS / R;  // steps of a tile and of a thread
     __shared__ int s_tile, s_wide;
