@@ -109,7 +109,8 @@ def measure(path, few=None):
 # passes; the finishing kernel's three costs; what each further workgroup of a CU adds to the prologues. The bounds
 # of the ratios keep q / rate[q] from falling and rate[q] at q or less.
 PAIRS = [(n, s) for n in LANES for s in LANES[n]]
-LOW = [0.02, 0.5] + [1, 0.3, 1, 0.85, 0.85, 0.85, 1, 0.85, 0.85, 0.85] * 3 + [0.2, 0.05] * 7 + [0.01, 0.05, 0.02] + [0] * 6
+LOW = ([0.02, 0.5] + [1, 0.3, 1, 0.85, 0.85, 0.85, 1, 0.85, 0.85, 0.85] * 3 + [0.2, 0.05] * 7 + [0.01, 0.05, 0.02] +
+       [0] * 6)
 HIGH = [0.6, 8] + [15, 12, 2, 1.5, 4 / 3, 1.5, 2, 1.5, 4 / 3, 1.5] * 3 + [8, 3] * 7 + [0.3, 3, 2] + [2] * 6
 START = [0.13, 2.5] + [5, 3, 1.5, 1.25, 1.1, 1.1, 1.3, 1.15, 1.1, 1.1] * 3 + [1, 0.4] * 7 + [0.08, 0.5, 0.2] + [0.2] * 6
 
@@ -185,10 +186,11 @@ def fit(path):
         num = lambda v: f"{v:.2f}"
         many = lambda v: ", ".join(map(num, v))
         fin = t["fin"] if bwd else (0, 0, 0)
-        print(f"constexpr CostModel {name} = {{\n    {t['fold']:.3f}, {num(t['launch'])},\n    {fin[0]:.3f}, {many(fin[1:])},")
+        print(f"constexpr CostModel {name} = {{\n    {t['fold']:.3f}, {num(t['launch'])},")
+        print(f"    {fin[0]:.3f}, {many(fin[1:])},")
         print("    {" + ",\n     ".join(
-            f"{{{many((t['main'][i], t['main_more'][i], t['carry'][i], t['carry_more'][i]))}, {{{many(t['rate'][i])}}}, "
-            f"{{{many(t['crate'][i])}}}}}" for i in range(3)) + "},")
+            f"{{{many([t[k][i] for k in ('main', 'main_more', 'carry', 'carry_more')])}, "
+            f"{{{many(t['rate'][i])}}}, {{{many(t['crate'][i])}}}}}" for i in range(3)) + "},")
         print("    {" + ",\n     ".join("{" + ", ".join(
             "{" + many(t["chunk"][PAIRS.index((n, s))]) + "}" if s in LANES[n] else "{0, 0}" for s in (1, 2, 4)) + "}"
             for n in LANES) + "}};", flush=True)
