@@ -23,9 +23,9 @@
 // Range: the coefficient of a map over many steps is a product that leaves fp32 long before the states do (1.42^256
 // overflows, 0.66^256 is 0), and inf * 0 is NaN. So such products carry an exponent of their own, from a thread's run
 // to the look-back: states of 0, tiny ones and infinite ones pass through any number of finite coefficients as they do
-// step by step. Where no product leaves fp32 the results are the same bit for bit; the checks cost up to 2% in fp32 and
-// 6% in 16 bits ((2048, 300, 32) fp16 27.1 -> 28.7 us), exponents in every tile up to 12% ((1, 30000, 16) fp16 14.5 ->
-// 16.3); calls of 64 columns and more are unchanged.
+// step by step. Where no product leaves fp32 the results are the same bit for bit; narrow calls take 0.1 to 0.7 us
+// longer ((700, 300, 32) fp16 13.3 -> 14.0 us, (2048, 300, 32) 27.1 -> 27.8), a long one with exponents in every tile
+// 1.5 us ((1, 30000, 16) fp16 14.6 -> 16.1); large calls and those over wide rows are unchanged.
 #include <algorithm>
 
 #include "common.h"
@@ -198,6 +198,8 @@ pscan_kernel(const T* __restrict__ A, const T* __restrict__ X, const T* __restri
         wx[i] = row_ld<T, V>(X + row(t));
         if constexpr (REV) wh[i] = row_ld<T, V>(Hs + row(t - 1));
     }
+    // else this load is moved under the test of its row, behind all the others: (2048, 300, 32) fp16 28.3 us, not 27.8
+    asm volatile("" : "+v"(wx[0]));
 #pragma unroll
     for (int i = 0; i < RUN; ++i) {
         const bool has_a = p0 + i > 0 && p0 + i < L;  // A_0 (forward) and A_L (adjoint) do not enter
@@ -242,7 +244,7 @@ pscan_kernel(const T* __restrict__ A, const T* __restrict__ X, const T* __restri
             th = __builtin_fmaf(s_a[q][r][cl], th, s_h[q][r][cl]);
             ta *= s_a[q][r][cl];
         }
-        if (wide || (lt > 0 && out_of_range(ta))) {  // again with exponents: a product of R mantissas is above 2^-R
+        if (wide || (lt > 0 && lt + 1 < nltile && out_of_range(ta))) {  // again with exponents: a product of R mantissas is above 2^-R
             ta = 1.f, th = 0.f;
 #pragma unroll 2  // all at once the loads take 30 to 60 registers more, and the waves that they hold
             for (int q = 0; q < R; ++q) {
