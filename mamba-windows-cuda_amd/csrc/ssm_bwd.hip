@@ -452,10 +452,16 @@ ssm_bwd_kernel(
 #pragma unroll
         for (int j = 0; j < SPL; ++j) am = __builtin_fmaxf(am, __builtin_fabsf(A2[j]));
         s_amax[c * AMS + g] = am;
-    } else {  // few loads, and this instance spills at the register limit: 154 us against 167 (B=8 L=2048 D=1536)
+    } else {
+        // Few loads, and this instance spills at the register limit: 154 us against 167 (B=8 L=2048 D=1536). Where the
+        // factor is applied, to the maximum or to each value (the same bound), moves what is spilled: with softplus fp32
+        // takes 222 us one way and 248 the other, fp16 235 and 223; with the gate fp32 369 and 387, fp16 211 and 203.
+        constexpr bool kAfter = sizeof(T) == 4;
 #pragma unroll
         for (int n = 0; n < NS; ++n)
-            lamax2 = __builtin_fmaxf(lamax2, __builtin_fabsf(ld(A + (int64_t)ld_d * NS + n)) * kLog2e);
+            lamax2 = __builtin_fmaxf(lamax2,
+                                     __builtin_fabsf(ld(A + (int64_t)ld_d * NS + n)) * (kAfter ? 1.f : kLog2e));
+        if constexpr (kAfter) lamax2 *= kLog2e;
     }
     const float lbias = XD && xf.delta_bias ? ld(static_cast<const T*>(xf.delta_bias) + ld_d) : 0.f;
     // d delta' / d delta (softplus) of the loader's elements, for the chunk being stored and the next
