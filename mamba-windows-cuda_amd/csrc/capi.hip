@@ -213,10 +213,19 @@ SegPlan split_plan(const SsmShape& s, bool bwd, int spl, int cap_main, int cap_c
 // of the gfx950 build), or, when no device can be queried, min(512 / VGPRs, 160 KiB / LDS) of the
 // N=16 instances.
 int cap_or(int queried, int fallback) { return queried > 0 ? queried : fallback; }
-int fwd_cap(int ns, int spl) { return cap_or(fwd_wgs_per_cu(ns, spl, 0), spl == 1 ? 7 : spl == 2 ? 3 : 1); }
-int fwd_carry_cap(int ns, int spl) { return cap_or(fwd_wgs_per_cu(ns, spl, 2), spl == 1 ? 8 : spl == 2 ? 6 : 4); }
-int bwd_cap(int ns, int spl) { return cap_or(bwd_wgs_per_cu(ns, spl, false), spl == 1 ? 4 : spl == 2 ? 3 : 1); }
-int bwd_carry_cap(int ns, int spl) { return cap_or(bwd_wgs_per_cu(ns, spl, true), spl == 1 ? 8 : spl == 2 ? 6 : 4); }
+int main_kernel(XfClass cls) { return cls == kXfClassOther ? kOccMain : kOccBoth + cls; }
+int fwd_cap(int ns, int spl, XfClass cls = kXfClassOther) {
+    return cap_or(fwd_wgs_per_cu(ns, spl, main_kernel(cls)), spl == 1 ? 7 : spl == 2 ? 3 : 1);
+}
+int bwd_cap(int ns, int spl, XfClass cls = kXfClassOther) {
+    return cap_or(bwd_wgs_per_cu(ns, spl, main_kernel(cls)), spl == 1 ? 4 : spl == 2 ? 3 : 1);
+}
+int fwd_carry_cap(int ns, int spl) {
+    return cap_or(fwd_wgs_per_cu(ns, spl, kOccCarry), spl == 1 ? 8 : spl == 2 ? 6 : 4);
+}
+int bwd_carry_cap(int ns, int spl) {
+    return cap_or(bwd_wgs_per_cu(ns, spl, kOccCarry), spl == 1 ? 8 : spl == 2 ? 6 : 4);
+}
 
 size_t carry_bytes(const SsmShape& s, const SegPlan& p) {
     return p.nseg > 1 ? align256((size_t)s.batch * p.ncar * s.dim * s.nstate * sizeof(float)) : 0;
@@ -328,6 +337,13 @@ double pass_us(int wgs, int chunks, int cap, double chunk, double prologue, doub
 int state_index(int ns) { return ns == 8 ? 0 : ns == 16 ? 1 : ns == 32 ? 2 : 3; }
 int lane_index(int spl) { return spl == 4 ? 2 : spl - 1; }
 
+// With both transforms the N=8 backward at two states per lane spills 88 bytes in its chunk loop: calls take 1.65 to 2
+// times those without (1.2 times at one state). From 1.5 to 1.7 the choice is within 3% of the fastest plan.
+bool spilling(const SsmShape& s, bool bwd, int spl, XfClass cls) {
+    return bwd && s.nstate == 8 && spl == 2 && cls != kXfClassOther;
+}
+constexpr double kSpilledChunk = 1.6;
+
 // Modelled plans of one shape and direction at one count of states per lane
 struct PlanCost {
     const SsmShape& s;
@@ -335,12 +351,13 @@ struct PlanCost {
     const bool bwd;
     const int si, wgs, cap_main, cap_carry;  // wgs: workgroups of one segment
     const double main_chunk, carry_chunk, fin, fin_rows;
-    PlanCost(const SsmShape& s_, bool bwd_, int spl)
+    PlanCost(const SsmShape& s_, bool bwd_, int spl, XfClass cls)
         : s(s_), m(bwd_ ? kBwdCost : kFwdCost), bwd(bwd_), si(lane_index(spl)),
           wgs((int)(s.batch * ((s.dim + cpb_of(s.nstate, spl) - 1) / cpb_of(s.nstate, spl)))),
-          cap_main(bwd ? bwd_cap(s.nstate, spl) : fwd_cap(s.nstate, spl)),
+          cap_main(bwd ? bwd_cap(s.nstate, spl, cls) : fwd_cap(s.nstate, spl, cls)),
           cap_carry(bwd ? bwd_carry_cap(s.nstate, spl) : fwd_carry_cap(s.nstate, spl)),
-          main_chunk(m.chunk[state_index(s.nstate)][si].main), carry_chunk(m.chunk[state_index(s.nstate)][si].carry),
+          main_chunk(m.chunk[state_index(s.nstate)][si].main * (spilling(s, bwd, spl, cls) ? kSpilledChunk : 1.0)),
+          carry_chunk(m.chunk[state_index(s.nstate)][si].carry),
           fin(m.fin_group * (wgs / (double)s.batch)), fin_rows(m.fin_rows) {}
     // the main pass and the finishing kernel of nseg segments of cps chunks
     double main_us(int nseg, int cps) const {
@@ -364,9 +381,9 @@ struct PlanCost {
 
 // The model's plan where it undercuts `p` clearly, else `p`. Never one whose carries need more scratch than `p`'s and
 // than the scratch of mwc_ssm_fwd_noalloc, so that no size which that entry point takes gets refused. (The backward's
-// partials follow its segments and states per lane: of 6,000 random shapes its workspace is at most 1.6 times that of
-// `p`, and under 0.8 times at 1,842.)
-SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
+// partials follow its segments and states per lane: of 6,000 random shapes its workspace is at most 1.9 times that of
+// `p`, over 1.2 times at 159 and under 0.8 times at 1,675.)
+SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p, XfClass cls) {
     const int64_t chunks = (s.seqlen + kCkptSteps - 1) / kCkptSteps;
     const int64_t w1 = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl));
     const auto& known = kFwdCost.chunk[state_index(s.nstate)];
@@ -374,7 +391,7 @@ SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
     if (w1 <= 0 || chunks < 2 || w1 >= (int64_t)kCUs * 3 / 2 || known[lane_index(p.spl)].main == 0) return p;
     const int nck = (int)chunks;
     SegPlan best = p;
-    const PlanCost own(s, bwd, p.spl);
+    const PlanCost own(s, bwd, p.spl, cls);
     double best_t = own.main_us(p.nseg, p.cps);
     if (p.nseg > 1)
         best_t += own.carry_us(p.ncar, p.cps / p.cfold, bwd ? p.ncar : (p.nseg - 1) * p.cfold);
@@ -382,7 +399,7 @@ SegPlan small_grid_plan(const SsmShape& s, bool bwd, const SegPlan& p) {
     const size_t most = std::max<size_t>(carry_bytes(s, p), MWC_NOALLOC_SCRATCH_BYTES / 2);
     for (int spl = 1; spl <= 4; spl *= 2) {
         if (known[lane_index(spl)].main == 0) continue;
-        const PlanCost c(s, bwd, spl);
+        const PlanCost c(s, bwd, spl, cls);
         for (int n : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48}) {
             const int per = (nck + n - 1) / n;
             if (n > 1 && per < 2) break;  // segments of one chunk run longer than modelled
@@ -439,22 +456,45 @@ SegPlan plan_rules(const SsmShape& s, bool bwd) {
     return h.nseg > 0 && (x_forced > 0 || th < t * 0.98) ? h : p;
 }
 
-// The plans of the shapes that this thread asked for last are kept, per direction (64 of them, one per slot): a call
+// A shape's plans, by the class of the call's instance. Both transforms take a wave of some main kernels' four states
+// per lane (16 bits: 247 VGPRs -> 258 in the N=32 backward), and a plan that fills two waves then takes two rounds:
+// (2, 2048, 2560) N=32 bf16 backward with both 317 us by the rules, 400 by the plan of the call without them.
+struct ShapePlans {
+    SegPlan p[3];
+};
+
+ShapePlans shape_plans(const SsmShape& s, bool bwd) {
+    const SegPlan rules = plan_rules(s, bwd);
+    ShapePlans r{{rules, rules, rules}};
+    if (rules.nfull > 0 || s.batch <= 0 || s.dim <= 0) return r;
+    const SegPlan p = r.p[0] = small_grid_plan(s, bwd, rules, kXfClassOther);
+    const int64_t wgs = s.batch * ((s.dim + cpb_of(s.nstate, p.spl) - 1) / cpb_of(s.nstate, p.spl)) * p.nseg;
+    for (XfClass cls : {kXfClassBoth16, kXfClassBoth32}) {  // where its grid fits, no other costs the class less
+        const int cap = bwd ? bwd_cap(s.nstate, p.spl, cls) : fwd_cap(s.nstate, p.spl, cls);
+        const bool same = wgs <= (int64_t)kCUs * cap && !spilling(s, bwd, p.spl, cls);
+        r.p[cls] = same ? p : small_grid_plan(s, bwd, rules, cls);
+    }
+    return r;
+}
+
+// The plans of the shapes that this thread asked for last are kept, per direction (64 shapes, one per slot): a call
 // asks for its plan three times, and a program for the same few shapes over and over. Overrides (tuning and tests) are
 // read on every call.
-SegPlan plan_dir(const SsmShape& s, bool bwd) {
+ShapePlans plan_dir(const SsmShape& s, bool bwd) {
     for (const char* e : {"MWC_SPL", "MWC_NSEG", "MWC_CFOLD", "MWC_NSPLIT"})
-        if (getenv(e) != nullptr) return plan_rules(s, bwd);
+        if (getenv(e) != nullptr) {
+            const SegPlan p = plan_rules(s, bwd);
+            return ShapePlans{{p, p, p}};
+        }
     struct Kept {
         SsmShape s{-1, -1, -1, 0};  // no shape
-        SegPlan p{};
+        ShapePlans p{};
     };
     static thread_local Kept kept[2][64];
     const uint64_t h = ((uint64_t)s.batch * 31 + (uint64_t)s.seqlen) * 1000003 + (uint64_t)s.dim * 127 + s.nstate;
     Kept& k = kept[bwd][(h * 0x9e3779b97f4a7c15ull) >> 58];
     if (k.s.nstate != s.nstate || k.s.batch != s.batch || k.s.seqlen != s.seqlen || k.s.dim != s.dim) {
-        const SegPlan p = plan_rules(s, bwd);
-        k.p = p.nfull > 0 ? p : small_grid_plan(s, bwd, p);
+        k.p = shape_plans(s, bwd);
         k.s = s;
     }
     return k.p;
@@ -462,23 +502,30 @@ SegPlan plan_dir(const SsmShape& s, bool bwd) {
 
 }  // namespace
 
-SegPlan plan_fwd(const SsmShape& s) { return plan_dir(s, false); }
+SegPlan plan_fwd(const SsmShape& s, XfClass cls) { return plan_dir(s, false).p[cls]; }
 
-SegPlan plan_bwd(const SsmShape& s) { return plan_dir(s, true); }
+SegPlan plan_bwd(const SsmShape& s, XfClass cls) { return plan_dir(s, true).p[cls]; }
 
+// Workspace sizes are the largest of the classes', so that one size serves a shape with and without transforms.
 size_t fwd_workspace_bytes(const SsmShape& s) {
-    // the segment carries when L is split
-    return 2 * carry_bytes(s, plan_fwd(s));
+    size_t n = 0;
+    for (const SegPlan& p : plan_dir(s, false).p) n = std::max(n, 2 * carry_bytes(s, p));  // when L is split
+    return n;
 }
 
-size_t bwd_workspace_bytes(const SsmShape& s) {
-    const SegPlan p = plan_bwd(s);
+static size_t bwd_bytes(const SsmShape& s, const SegPlan& p) {
     size_t n = align256((size_t)bwd_groups(s, s.nstate, p.spl) * s.batch * s.seqlen * 2 * s.nstate *
                         sizeof(float));                                                          // dB/dC
     n += align256((size_t)p.nseg * s.batch * s.dim * s.nstate * sizeof(float));                  // dA
     n += align256((size_t)p.nseg * s.batch * s.dim * sizeof(float));                                // dD
     n += align256((size_t)p.nseg * s.batch * s.dim * sizeof(float));                                // d bias
     n += 2 * carry_bytes(s, p);
+    return n;
+}
+
+size_t bwd_workspace_bytes(const SsmShape& s) {
+    size_t n = 0;
+    for (const SegPlan& p : plan_dir(s, true).p) n = std::max(n, bwd_bytes(s, p));
     return n;
 }
 
@@ -549,6 +596,11 @@ size_t mwc_ssm_bwd_workspace_size(int64_t batch, int64_t seqlen, int64_t dim, in
     return mwc::bwd_workspace_bytes({batch, seqlen, dim, (int)dstate});
 }
 
+static mwc::XfClass xf_class(int dtype, const void* delta_bias, int delta_softplus, bool gate) {
+    if (!gate || (delta_bias == nullptr && delta_softplus == 0)) return mwc::kXfClassOther;
+    return dtype == MWC_DTYPE_F32 ? mwc::kXfClassBoth32 : mwc::kXfClassBoth16;
+}
+
 // The forward's one body: validation, workspace check and launch. With `scratch_only`, the segment
 // carries live in this device's static scratch array (mwc_ssm_fwd_noalloc) instead of a caller
 // workspace; sizes whose carries exceed it are rejected before anything is enqueued.
@@ -609,7 +661,8 @@ static int fwd_impl(int dtype, const void* u, const void* delta, const void* A, 
     }
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MWC_ERR_WORKSPACE, "forward workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
-    const mwc::SegPlan p = mwc::plan_fwd(s);
+    const bool gate = z != nullptr && out_z != nullptr;
+    const mwc::SegPlan p = mwc::plan_fwd(s, xf_class(dtype, delta_bias, delta_softplus, gate));
     float* car_h = (float*)workspace;
     float* car_x = (float*)((char*)workspace + need / 2);
     const mwc::FwdArgs a{u, delta, A, B_ssm, C_ssm, D_ssm, h_prev, out, h_last, ckpt, car_h, car_x,
@@ -655,7 +708,7 @@ int mwc_ssm_bwd_ex(int dtype, const void* u, const void* delta, const void* A, c
         return fail(MWC_ERR_WORKSPACE, "backward workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
     hipStream_t st = (hipStream_t)stream;
     char* w = (char*)workspace;
-    const mwc::SegPlan p = mwc::plan_bwd(s);
+    const mwc::SegPlan p = mwc::plan_bwd(s, xf_class(dtype, delta_bias, delta_softplus, z != nullptr));
     const int ngrp = mwc::bwd_groups(s, s.nstate, p.spl);
     float* dbc_part = (float*)w;
     w += align256((size_t)ngrp * batch * seqlen * 2 * dstate * sizeof(float));

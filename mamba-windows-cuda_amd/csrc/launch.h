@@ -76,12 +76,17 @@ __device__ __forceinline__ WorkItem carry_item(int lid, int rows, int nfull) {
     const int first = nfull > 0 ? nfull : 0, n = rows - first;
     return WorkItem{first + lid % n, lid / n, false};
 }
-SegPlan plan_fwd(const SsmShape& s);
-SegPlan plan_bwd(const SsmShape& s);
+// The instance that a call runs, where that matters to its plan: with both transforms fewer waves of some main kernels
+// fit a SIMD, and which ones depends on the storage type.
+enum XfClass { kXfClassOther = 0, kXfClassBoth16 = 1, kXfClassBoth32 = 2 };
+SegPlan plan_fwd(const SsmShape& s, XfClass cls);
+SegPlan plan_bwd(const SsmShape& s, XfClass cls);
 // Workgroups per CU of a lane-group kernel instance (the HIP runtime's occupancy query, cached), or 0 when
-// no device can be queried. fwd mode: 0 main, 1 state-only, 2 carry.
-int fwd_wgs_per_cu(int ns, int spl, int mode);
-int bwd_wgs_per_cu(int ns, int spl, bool carry);
+// no device can be queried. which: kOccMain, kOccState (forward only), kOccCarry, or kOccBoth + the class of a main
+// kernel with both transforms.
+constexpr int kOccMain = 0, kOccState = 1, kOccCarry = 2, kOccBoth = 2;
+int fwd_wgs_per_cu(int ns, int spl, int which);
+int bwd_wgs_per_cu(int ns, int spl, int which);
 
 // Workspace carve-up (bytes, 256-aligned pieces).
 size_t fwd_workspace_bytes(const SsmShape& s);

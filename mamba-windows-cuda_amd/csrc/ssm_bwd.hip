@@ -870,17 +870,19 @@ __global__ void __launch_bounds__(256) bwd_finish_kernel(const float* __restrict
     }
 }
 
-int bwd_wgs_per_cu(int ns, int spl, bool carry) {
-    // as fwd_wgs_per_cu: the fp16, transform-free instance's occupancy, queried once; 0 if unknown
-    static std::atomic<int> cache[4][3][2];
+int bwd_wgs_per_cu(int ns, int spl, int which) {  // as fwd_wgs_per_cu
+    static std::atomic<int> cache[4][3][5];
     const int ni = ns == 8 ? 0 : ns == 16 ? 1 : ns == 32 ? 2 : 3, si = spl == 1 ? 0 : spl == 2 ? 1 : 2;
-    int v = cache[ni][si][carry].load(std::memory_order_relaxed);
+    int v = cache[ni][si][which].load(std::memory_order_relaxed);
     if (v != 0) return v < 0 ? 0 : v;
     const void* k = nullptr;
 #define MWC_BWD_K(N, S)                                                                                   \
     if (ns == N && spl == S)                                                                              \
-        k = carry ? reinterpret_cast<const void*>(&ssm_bwd_carry_kernel<half_t, N, S, 0>)                 \
-                  : reinterpret_cast<const void*>(&ssm_bwd_kernel<half_t, N, S, 0>);
+        k = which == kOccCarry  ? reinterpret_cast<const void*>(&ssm_bwd_carry_kernel<half_t, N, S, 0>)   \
+            : which == kOccMain ? reinterpret_cast<const void*>(&ssm_bwd_kernel<half_t, N, S, 0>)         \
+            : which == kOccBoth + kXfClassBoth16                                                          \
+                ? reinterpret_cast<const void*>(&ssm_bwd_kernel<half_t, N, S, kXfDelta | kXfGate>)        \
+                : reinterpret_cast<const void*>(&ssm_bwd_kernel<float, N, S, kXfDelta | kXfGate>);
     MWC_FOR_EACH_LANE_GROUP(MWC_BWD_K)
 #undef MWC_BWD_K
     int n = 0;
@@ -888,7 +890,7 @@ int bwd_wgs_per_cu(int ns, int spl, bool carry) {
         (void)hipGetLastError();
         n = -1;
     }
-    cache[ni][si][carry].store(n, std::memory_order_relaxed);
+    cache[ni][si][which].store(n, std::memory_order_relaxed);
     return n < 0 ? 0 : n;
 }
 

@@ -430,19 +430,22 @@ static hipError_t fwd_inst(const FwdArgs& a, const SsmShape& s, hipStream_t st) 
     }
 }
 
-int fwd_wgs_per_cu(int ns, int spl, int mode) {
-    // the runtime's occupancy of the fp16, transform-free instance (registers and LDS differ little
-    // across dtypes and transforms), queried once per (N, SPL, mode); 0 when it cannot be queried
-    static std::atomic<int> cache[4][3][3];
+int fwd_wgs_per_cu(int ns, int spl, int which) {
+    // the runtime's occupancy of the fp16, transform-free instance (registers and LDS differ little across dtypes and
+    // single transforms) or of a main kernel with both, queried once per (N, SPL, which); 0 when it cannot be queried
+    static std::atomic<int> cache[4][3][5];
     const int ni = ns == 8 ? 0 : ns == 16 ? 1 : ns == 32 ? 2 : 3, si = spl == 1 ? 0 : spl == 2 ? 1 : 2;
-    int v = cache[ni][si][mode].load(std::memory_order_relaxed);
+    int v = cache[ni][si][which].load(std::memory_order_relaxed);
     if (v != 0) return v < 0 ? 0 : v;
     const void* k = nullptr;
 #define MWC_FWD_K(N, S)                                                                                         \
     if (ns == N && spl == S)                                                                                    \
-        k = mode == kCarry   ? reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kCarry, 0>)        \
-            : mode == kState ? reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kState, 0>)        \
-                             : reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kMain, 0>);
+        k = which == kOccCarry   ? reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kCarry, 0>)      \
+            : which == kOccState ? reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kState, 0>)      \
+            : which == kOccMain  ? reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kMain, 0>)       \
+            : which == kOccBoth + kXfClassBoth16                                                                \
+                ? reinterpret_cast<const void*>(&ssm_fwd_kernel<half_t, N, S, kMain, kXfDelta | kXfGate>)       \
+                : reinterpret_cast<const void*>(&ssm_fwd_kernel<float, N, S, kMain, kXfDelta | kXfGate>);
     MWC_FOR_EACH_LANE_GROUP(MWC_FWD_K)
 #undef MWC_FWD_K
     int n = 0;
@@ -450,7 +453,7 @@ int fwd_wgs_per_cu(int ns, int spl, int mode) {
         (void)hipGetLastError();
         n = -1;
     }
-    cache[ni][si][mode].store(n, std::memory_order_relaxed);
+    cache[ni][si][which].store(n, std::memory_order_relaxed);
     return n < 0 ? 0 : n;
 }
 

@@ -283,7 +283,7 @@ def test_planner_small_grids_against_the_rules(monkeypatch):
     scratch = 32 << 20  # MWC_NOALLOC_SCRATCH_BYTES
     for s in shapes:
         assert model[s][0] <= max(rules[s][0], scratch), s
-        assert model[s][1] <= 1.75 * rules[s][1], s
+        assert model[s][1] <= 2 * rules[s][1], s
     monkeypatch.setenv("MWC_NSEG", "1")
     for s, spl in short.items():
         monkeypatch.setenv("MWC_SPL", str(spl))

@@ -209,6 +209,25 @@ def test_planner_small_grids(dev, monkeypatch, idx):
     _run_case(dev, monkeypatch, 40000 + idx, conditioned=True, c=c)
 
 
+# The same with both transforms, whose plan is one of its own where they change a kernel's occupancy (16 bits at N=32
+# and 64) or spill (N=8); fp32 beside them.
+BOTH_CASES = [dict(B=2, L=300, D=1100, n=8, dtype=torch.float16, seed=611),
+              dict(B=1, L=500, D=1700, n=8, dtype=torch.float32, seed=612),
+              dict(B=1, L=700, D=1500, n=32, dtype=torch.bfloat16, seed=613),
+              dict(B=2, L=333, D=900, n=32, dtype=torch.float32, seed=614),
+              dict(B=2, L=260, D=1100, n=64, dtype=torch.float16, seed=615),
+              dict(B=1, L=1024, D=256, n=16, dtype=torch.float16, seed=616)]
+
+
+@pytest.mark.parametrize("idx", range(len(BOTH_CASES)))
+def test_planner_small_grids_with_both_transforms(dev, monkeypatch, idx):
+    c = dict(with_h=True, bias=True, softplus=True, gate=True, spl=None, nseg=None, cfold=None, lvl=idx % 2,
+             **BOTH_CASES[idx])
+    for var in ("MWC_SPL", "MWC_NSEG", "MWC_CFOLD", "MWC_NSPLIT"):
+        monkeypatch.delenv(var, raising=False)
+    _run_case(dev, monkeypatch, 50000 + idx, conditioned=True, c=c)
+
+
 @pytest.mark.parametrize("idx", CONDITIONED)
 def test_conditioned_case(dev, monkeypatch, idx):
     _run_case(dev, monkeypatch, idx, conditioned=True)
